@@ -1,5 +1,8 @@
 // Conv1d / ConvTranspose1d forward, input-grad and weight-grad on gfx950 as
-// implicit GEMMs on FP32 MFMA (v_mfma_f32_32x32x2_f32).
+// implicit GEMMs on the matrix units, in float precision throughout: the
+// forwards and strided correlations on FP32 MFMA (v_mfma_f32_32x32x2_f32), the
+// stride-1 input grads on bf16 MFMA with every float split exactly into three
+// bf16 terms (split_gemm).
 //
 // Forward family (one kernel, `conv_gemm`):
 //   Y[n, m, q] = sum_{c, t} A[(c, t), m] * X[n, c, q*s + t*d - p]
@@ -85,6 +88,7 @@ struct GemmArgs {
     int ybuf;                // (C_out + BM) * L_y * 4 < 2^31: the epilogue addresses Y through a descriptor
     // octet mode (corr_gemm): K chunk = one input-channel octet x up to G taps
     int G, n_tg, n_oct, span8;  // taps per chunk, tap groups, octets, staged positions
+    int n_c16;               // split_gemm: 16-channel chunks (G taps at most each, n_tg tap groups); 0: another kernel
     int quad;                // conv_gemm_q: weights packed in quads of k-steps (stride 1, k = KT)
     // Output placement (polyphase transposed convs): every column lands y_off
     // positions on (a left pad of the output rows, whose length L_y counts
@@ -969,13 +973,7 @@ void conv_gemm_q(GemmArgs g) {
     asm volatile("" : "+s"(te));
     TileGeo Te;
     decode_tile(g, te, Te);
-    if constexpr (EPI == QEPI_ADAIN_BWD) {
-        if (part < 0) {  // uniform per block
-            store_tile_adain(g, Te, acc, wm, wn, hi, l32, smem);
-        } else {
-            store_tile(g, Te, te, part, acc, wm, wn, hi, l32);
-        }
-    } else if constexpr (EPI == QEPI_STATS) {
+    if constexpr (EPI == QEPI_STATS) {
         if (part < 0)
             store_tile_stats(g, Te, acc, wm, wn, hi, l32);
         else
@@ -1126,6 +1124,260 @@ void corr_gemm(GemmArgs g) {
     }
 
     store_tile(g, T, tile, part, acc, wm, wn, hi, l32);
+}
+
+// Stride-1 correlation on the bf16 matrix units at float precision: every
+// float operand is split exactly into three bf16 terms, x = h + m + l (8 + 8 +
+// 8 significant bits), and a product is the six bf16 products of order up to
+// 2^-16, accumulated in float: h h' in one accumulator, m h' + h m' + m m' +
+// l h' + h l' in a second that is added once at the end (the dropped terms lie
+// below 2^-26 of the product). The two accumulators keep the matrix unit's
+// rounding of the small terms off the large sum: against double, over K = 16
+// .. 32768 random terms, 0.3-0.45 of v_mfma_f32_32x32x2's error, and none of
+// the downward bias that six products into one accumulator show (-8e-8 of the
+// rms at K = 1408). Bound: MFMA. Six v_mfma_f32_32x32x16_bf16 do 16 channels
+// where the float unit takes eight instructions of twice the cycles: measured
+// ceilings 1461-1686 / 6 = 244-281 TFLOP/s (the power limit, not the 2.5
+// PFLOP/s issue rate) against 140.
+//
+// K runs over (16-channel chunk, tap). A chunk's input window [16][span] is
+// loaded as floats into registers while the previous chunk is multiplied,
+// split once, and stored channels-last in three LDS planes [position][16]: a
+// tap is then a shift by whole 32-byte rows, so every fragment is one aligned
+// conflict-free ds_read_b128 whatever the dilation. The weights come split
+// and in fragment order from pack_split ([m_tile][step][plane][32-row block]
+// [lane][8], 12 KB per step of 128 rows), straight from L2 into registers one
+// step ahead: they would take 12 KB of LDS and a barrier per step, and every
+// block of an XCD reads the same panel at about the same time.
+//
+// KT > 0: the tap count, all taps in one chunk. KT = 0: k at run time, chunks
+// of up to G taps so that any dilation's window fits.
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int SPLIT_STEP = 3 * BM * 16 / 2;  // floats of panel per (128 rows, step): three planes of 128 x 16 bf16
+constexpr int SPLIT_SPAN = 256;              // staged positions at most (two 8-channel items per thread)
+
+// x = h + m + l exactly (round to nearest each time, the last remainder fits).
+__device__ inline void split3(float x, __bf16& h, __bf16& m, __bf16& l) {
+    h = static_cast<__bf16>(x);
+    const float r = x - static_cast<float>(h);
+    m = static_cast<__bf16>(r);
+    l = static_cast<__bf16>(r - static_cast<float>(m));
+}
+
+__device__ inline void split_mma(const bf16x8 (&a)[3][2], const bf16x8 (&b)[3][2], f32x16 (&hh)[2][2],
+                                 f32x16 (&lo)[2][2]) {
+#define KDEC_SPLIT_MMA(ACC, I, J)                                                                       \
+    _Pragma("unroll") for (int tm = 0; tm < 2; ++tm) _Pragma("unroll") for (int tn = 0; tn < 2; ++tn)   \
+        ACC[tm][tn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[I][tm], b[J][tn], ACC[tm][tn], 0, 0, 0);
+    KDEC_SPLIT_MMA(lo, 0, 2)
+    KDEC_SPLIT_MMA(lo, 2, 0)
+    KDEC_SPLIT_MMA(lo, 1, 1)
+    KDEC_SPLIT_MMA(lo, 0, 1)
+    KDEC_SPLIT_MMA(lo, 1, 0)
+    KDEC_SPLIT_MMA(hh, 0, 0)
+#undef KDEC_SPLIT_MMA
+}
+
+template <int KT, int EPI>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2)))
+void split_gemm(GemmArgs g) {
+    extern __shared__ float smem[];
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave & 1, wn = wave >> 1;
+    const int l32 = lane & 31, hi = lane >> 5;
+
+    int tile, part;
+    if (!block_work(g, tile, part)) return;  // uniform per block
+    TileGeo T;
+    decode_tile(g, tile, T);
+    if (T.q0 >= T.n_q) return;  // uniform per block
+    const int k = KT > 0 ? KT : T.k, d = T.d;
+    const int G = KT > 0 ? KT : g.G, n_tg = KT > 0 ? 1 : g.n_tg;
+    const int span = BN + (G - 1) * d;  // <= SPLIT_SPAN (run_gemm)
+    const int stage = 3 * span * 32;    // bytes
+    char* lds = reinterpret_cast<char*>(smem);
+
+    const int nchunks = g.n_c16 * n_tg;
+    const int nparts = part < 0 ? 1 : g.fsplit;
+    const int pp = part < 0 ? 0 : part;
+    const int ch0 = pp * nchunks / nparts;
+    const int ch1 = (pp + 1) * nchunks / nparts;
+
+    // Staging items: (position, channel octet) = (e >> 1, e & 1), e = tid and
+    // tid + 256; an item's eight channels are one 16-byte store per plane at
+    // byte 16 e of it.
+    const __amdgpu_buffer_rsrc_t xrs = uniform_rsrc(g.X + static_cast<long>(T.b) * g.x_bs, g.C_in * g.L_in * 4);
+    const int rowB = g.L_in * 4;
+    const bool two = wave * 64 + NT < 2 * span;  // wave-uniform: a second item
+    float xr[2][8];
+    auto load_item = [&](int i, int c16, int p0) {
+        const int e = tid + i * NT;
+        const int pos = p0 + (e >> 1);
+        // past the row: an offset past the buffer reads 0; so do channels past C_in
+        unsigned off = pos >= 0 && pos < g.L_in && e < 2 * span
+                           ? static_cast<unsigned>((c16 * 16 + (e & 1) * 8) * rowB + pos * 4) : 0x80000000u;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            xr[i][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrs, static_cast<int>(off), 0, 0));
+            off += rowB;
+        }
+    };
+    auto load_x = [&](int ch) {
+        const int c16 = ch / n_tg, tg = ch - c16 * n_tg;
+        const int p0 = T.q0 - T.p + tg * G * d;
+        load_item(0, c16, p0);
+        if (two) load_item(1, c16, p0);
+    };
+    auto store_item = [&](int i, int buf) {
+        const int e = tid + i * NT;
+        bf16x8 h, m, l;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            __bf16 a, b, c;
+            split3(xr[i][j], a, b, c);
+            h[j] = a;
+            m[j] = b;
+            l[j] = c;
+        }
+        if (e < 2 * span) {
+            char* p = lds + buf * stage + e * 16;
+            *reinterpret_cast<bf16x8*>(p) = h;
+            *reinterpret_cast<bf16x8*>(p + span * 32) = m;
+            *reinterpret_cast<bf16x8*>(p + 2 * span * 32) = l;
+        }
+    };
+    auto store_x = [&](int buf) {
+        store_item(0, buf);
+        if (two) store_item(1, buf);
+    };
+
+    // Weight fragments of step s (chunk-major, then tap): plane p, row block 2 wm + tm.
+    const int nsteps = g.n_c16 * k;
+    const float* Ap = T.A + static_cast<long>(T.m0 / BM) * nsteps * SPLIT_STEP;
+    const int a_lane = wm * 512 + lane * 4;  // floats
+    auto load_a = [&](int s, bf16x8 (&a)[3][2]) {
+        const float* p = Ap + static_cast<long>(s) * SPLIT_STEP;
+#pragma unroll
+        for (int pl = 0; pl < 3; ++pl)
+#pragma unroll
+            for (int tm = 0; tm < 2; ++tm)
+                a[pl][tm] = *reinterpret_cast<const bf16x8*>(p + pl * 1024 + tm * 256 + a_lane);
+    };
+
+    f32x16 acc[2][2], lo[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = lo[i][j][e] = 0.0f;
+
+    const bool live = T.q0 + wn * 64 < T.n_q;  // wave-uniform: some column is stored
+    const int s_end = (ch1 / n_tg) * k + (ch1 % n_tg) * G;
+    int s = (ch0 / n_tg) * k + (ch0 % n_tg) * G;
+    bf16x8 a[3][2];
+    if (ch0 < ch1) {
+        load_x(ch0);
+        if (live) load_a(s, a);
+        store_x(0);
+    }
+    __syncthreads();
+    const int b_lane = (wn * 64 + l32) * 32 + hi * 16;
+    for (int ch = ch0; ch < ch1; ++ch) {
+        const int buf = (ch - ch0) & 1;
+        if (ch + 1 < ch1) load_x(ch + 1);
+        if (live) {
+            const char* bp = lds + buf * stage + b_lane;
+            const int nt = KT > 0 ? KT : min(G, k - (ch % n_tg) * G);
+#pragma unroll
+            for (int t = 0; t < nt; ++t) {
+                bf16x8 an[3][2], b[3][2];
+                ++s;
+                load_a(min(s, s_end - 1), an);
+#pragma unroll
+                for (int pl = 2; pl >= 0; --pl)
+#pragma unroll
+                    for (int tn = 0; tn < 2; ++tn)
+                        b[pl][tn] = *reinterpret_cast<const bf16x8*>(bp + pl * span * 32 + tn * 1024);
+                split_mma(a, b, acc, lo);
+#pragma unroll
+                for (int pl = 0; pl < 3; ++pl)
+#pragma unroll
+                    for (int tm = 0; tm < 2; ++tm) a[pl][tm] = an[pl][tm];
+                bp += d * 32;
+            }
+        }
+        if (ch + 1 < ch1) store_x(buf ^ 1);
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] += lo[i][j][e];
+
+    // An infinity splits as inf + NaN + NaN, a float above the largest bf16
+    // likewise, and the matrix unit reads subnormal bf16 as zero, so the lower
+    // terms of operands under 2^-110 are lost. A wave with a column that is
+    // not finite, or not zero yet under 2^-90, forms its sums again on the
+    // float unit from the unsplit operands: such inputs give what they give
+    // there.
+    float mag = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) mag += fabsf(acc[i][j][e]);
+    if (live && __any(!(mag <= 3.4028235e38f) || (mag > 0.0f && mag < 0x1p-90f))) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+        for (int ch = ch0; ch < ch1; ++ch) {
+            const int c16 = ch / n_tg, tg = ch - c16 * n_tg;
+            const int t1 = min(k, (tg + 1) * G);
+            for (int t = tg * G; t < t1; ++t) {
+                load_a(c16 * k + t, a);
+                for (int j = 0; j < 8; ++j) {
+                    float av[2], bv[2];
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        av[u] = static_cast<float>(a[0][u][j]) +
+                                (static_cast<float>(a[1][u][j]) + static_cast<float>(a[2][u][j]));
+                        const int pos = T.q0 + wn * 64 + u * 32 + l32 - T.p + t * d;
+                        const unsigned off = pos >= 0 && pos < g.L_in
+                                                 ? static_cast<unsigned>((c16 * 16 + hi * 8 + j) * rowB + pos * 4)
+                                                 : 0x80000000u;
+                        bv[u] = __builtin_bit_cast(
+                            float, __builtin_amdgcn_raw_buffer_load_b32(xrs, static_cast<int>(off), 0, 0));
+                    }
+#pragma unroll
+                    for (int tm = 0; tm < 2; ++tm)
+#pragma unroll
+                        for (int tn = 0; tn < 2; ++tn)
+                            acc[tm][tn] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[tm], bv[tn], acc[tm][tn], 0, 0, 0);
+                }
+            }
+        }
+    }
+
+    if constexpr (EPI == QEPI_ADAIN_BWD) {
+        if (part < 0) {  // uniform per block
+            store_tile_adain(g, T, acc, wm, wn, hi, l32, smem);
+        } else {
+            store_tile(g, T, tile, part, acc, wm, wn, hi, l32);
+        }
+    } else {
+        store_tile(g, T, tile, part, acc, wm, wn, hi, l32);
+    }
 }
 
 // Split tiles: Y = scale * (sum of the parts in order + bias + R) + beta * Y.
@@ -1406,33 +1658,14 @@ __global__ void pack_fwd(const float* W, float* A, int C_in, int C_out, int k,
     }
 }
 
-// conv1d input-grad (stride 1): the correlation over dY (C_out channels) with
-// A[(co, t'), ci] = W[co, ci*k + (k-1-t')]
-__global__ void pack_dgrad(const float* W, float* A, int C_in, int C_out, int k,
-                           int cout_pad, int m_pad, int CK) {
-    const long total = static_cast<long>(cout_pad) * k * m_pad;
-    for (long i = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x; i < total;
-         i += static_cast<long>(gridDim.x) * blockDim.x) {
-        const int m = static_cast<int>(i % m_pad);  // ci
-        int c, t;                                   // c = co
-        panel_row(i / m_pad, CK, k, c, t);
-        float v = 0.0f;
-        if (m < C_in && c < C_out) v = W[(static_cast<long>(c) * C_in + m) * k + (k - 1 - t)];
-        A[i] = v;
-    }
-}
-
 // The quad panel of conv_gemm_q: A[m_tile][chunk][quad][hi][128][4], element
 // j of (quad g, hi, m) being packed row r = 2(4g + j) + hi of the chunk, i.e.
 // tap r / CK of channel chunk*CK + r % CK; zero past the chunk's CK*k/2
-// k-steps, past the channels or past the output rows. mode 0: conv1d forward
-// (A[(ci, t), co] = W[co, ci*k + t]); mode 1: conv1d input-grad at stride 1
-// (A[(co, t'), ci] = W[co, ci*k + k-1-t']). One thread writes one 16-B run.
-__global__ void pack_quad(const float* W, float* A, int mode, int C_in, int C_out, int k, int CK, int nchunks,
+// k-steps, past the channels or past the output rows (A[(ci, t), co] =
+// W[co, ci*k + t]). One thread writes one 16-B run.
+__global__ void pack_quad(const float* W, float* A, int C_in, int C_out, int k, int CK, int nchunks,
                           int Q, long total4) {
     const int S = CK * k / 2;
-    const int Cg = mode == 0 ? C_in : C_out;   // GEMM input channels
-    const int Mg = mode == 0 ? C_out : C_in;   // GEMM output rows
     for (long e = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x; e < total4;
          e += static_cast<long>(gridDim.x) * blockDim.x) {
         const int ml = static_cast<int>(e % BM);
@@ -1450,9 +1683,7 @@ __global__ void pack_quad(const float* W, float* A, int mode, int C_in, int C_ou
             const int r = 2 * u + hi;
             const int t = r / CK, c = ch * CK + r % CK;
             float x = 0.0f;
-            if (u < S && c < Cg && m < Mg)
-                x = mode == 0 ? W[(static_cast<long>(m) * C_in + c) * k + t]
-                              : W[(static_cast<long>(c) * C_in + m) * k + (k - 1 - t)];
+            if (u < S && c < C_in && m < C_out) x = W[(static_cast<long>(m) * C_in + c) * k + t];
             v[j] = x;
         }
         reinterpret_cast<float4*>(A)[e] = make_float4(v[0], v[1], v[2], v[3]);
@@ -1516,35 +1747,6 @@ __global__ __launch_bounds__(256) void pack_rows_t(const float* W, float* A, int
     }
 }
 
-// A[panel_index(c, t)][m] = W[c][m*k + k-1-t] (0 unless m < C_in, c < C_out):
-// the conv1d input-grad panel. Each wave takes one output channel c and a
-// 64-column m slice: it reads that slice's contiguous 64*k floats of W[c]
-// into LDS, then writes its k panel rows along m. Grid (cdiv(cpad, 4),
-// m_pad / 64), dynamic LDS 4 * 64 * k floats; cpad a multiple of CK.
-__global__ __launch_bounds__(256) void pack_dgrad_t(const float* W, float* A, int C_in, int C_out, int k,
-                                                    int cpad, int m_pad, int CK) {
-    extern __shared__ float seg_all[];
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    const int c = blockIdx.x * 4 + ty, m0 = blockIdx.y * 64;
-    float* seg = seg_all + ty * 64 * k;
-    const long base = static_cast<long>(c) * C_in * k + static_cast<long>(m0) * k;
-    const long lim = static_cast<long>(C_in) * k;  // valid part of row c
-    // k <= 32: a fixed trip count, unrolled, so the loads overlap
-    float v[32];
-#pragma unroll
-    for (int r = 0; r < 32; ++r) {
-        const int e = tx + 64 * r;
-        v[r] = (r < k && c < C_out && static_cast<long>(m0) * k + e < lim) ? W[base + e] : 0.0f;
-    }
-#pragma unroll
-    for (int r = 0; r < 32; ++r)
-        if (r < k) seg[tx + 64 * r] = v[r];
-    __syncthreads();
-    if (c >= cpad) return;
-    for (int t = 0; t < k; ++t)
-        A[panel_index(c, t, CK, k) * m_pad + m0 + tx] = seg[tx * k + (k - 1 - t)];
-}
-
 // conv-transpose forward, phase r of s: tap t' of kt covers original tap
 // t = r + (kt-1-t')*s.  A_r[(ci, t'), co] = W[ci, co*k + t] (0 if t >= k)
 __global__ void pack_convt_fwd(const float* W, float* A, int C_in, int C_out,
@@ -1568,8 +1770,7 @@ __global__ void pack_convt_fwd(const float* W, float* A, int C_in, int C_out,
 // corr_gemm panel [o][t][h][m_pad][4] for channel c = 8o + 4h + e and tap
 // t < kt (per phase, phase_stride floats each). `mode` is the weight map:
 // 0 conv forward            A[(c, t), m] = W[m, c*k + t]       (m < C_out, c < C_in)
-// 1 conv input-grad         A[(c, t), m] = W[c, m*k + k-1-t]   (m < C_in, c < C_out)
-// 2 conv-transpose forward, phase r of s: tap t covers original tap
+// 1 conv-transpose forward, phase r of s: tap t covers original tap
 //   r + (kt-1-t)*s, A_r[(c, t), m] = W[c, m*k + that] or 0   (m < C_out, c < C_in)
 __global__ void pack_octet(const float* W, float* A, int mode, int C_in, int C_out, int k, int s, int kt,
                            int m_pad, int phase_stride, int n_phase) {
@@ -1591,13 +1792,57 @@ __global__ void pack_octet(const float* W, float* A, int mode, int C_in, int C_o
         float v = 0.0f;
         if (mode == 0) {
             if (m < C_out && c < C_in) v = W[(m * C_in + c) * k + t];
-        } else if (mode == 1) {
-            if (m < C_in && c < C_out) v = W[(c * C_in + m) * k + (k - 1 - t)];
         } else {
             const int tt = static_cast<int>(r) + (kt - 1 - t) * s;
             if (m < C_out && c < C_in && tt < k) v = W[(c * C_out + m) * k + tt];
         }
         A[i] = v;
+    }
+}
+
+// split_gemm's weight panel [m_tile][step = c16*k + t][plane][32-row block]
+// [lane][8] of a conv1d input-grad, A[(co, t), ci] = W[co, ci*k + k-1-t]: lane
+// (hi, l32) of block mb holds row ci = 32 mb + l32 of the tile, channels co =
+// 16 c16 + 8 hi + j, split in three bf16 planes; zero past either. One thread
+// per (step, block, lane). A weight that is not finite, or rounds past bf16's
+// range, keeps h + m + l = w (h truncated, or m = l = 0); one under 2^-110
+// keeps it to 2^-133, bf16's smallest step.
+__global__ void pack_split(const float* W, float* A, int C_in, int C_out, int k, int nsteps, long total) {
+    for (long i = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x; i < total;
+         i += static_cast<long>(gridDim.x) * blockDim.x) {
+        const unsigned iu = static_cast<unsigned>(i);  // total < 2^31 (the host's check of the panel size)
+        const int lane = iu & 63, mb = (iu >> 6) & 3;
+        const unsigned rest = iu >> 8;
+        const unsigned st = rest % static_cast<unsigned>(nsteps);
+        const int mt = static_cast<int>(rest / static_cast<unsigned>(nsteps));
+        const int c16 = static_cast<int>(st) / k, t = static_cast<int>(st) - c16 * k;
+        const int m = mt * BM + mb * 32 + (lane & 31);
+        const int c0 = c16 * 16 + (lane >> 5) * 8;
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int c = c0 + j;
+            v[j] = m < C_in && c < C_out ? W[(static_cast<long>(c) * C_in + m) * k + (k - 1 - t)] : 0.0f;
+        }
+        bf16x8 p[3];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            __bf16 h, q, l;
+            split3(v[j], h, q, l);
+            if (!(fabsf(static_cast<float>(h)) <= 3.4e38f)) {
+                const float tr = __uint_as_float(__float_as_uint(v[j]) & 0xffff0000u);
+                const bool fin = fabsf(v[j]) <= 3.4028235e38f;
+                h = static_cast<__bf16>(v[j] != v[j] ? v[j] : tr);
+                q = static_cast<__bf16>(fin ? v[j] - tr : 0.0f);
+                l = static_cast<__bf16>(fin ? (v[j] - tr) - static_cast<float>(q) : 0.0f);
+            }
+            p[0][j] = h;
+            p[1][j] = q;
+            p[2][j] = l;
+        }
+        float* o = A + static_cast<long>(rest) * SPLIT_STEP + mb * 256 + lane * 4;
+#pragma unroll
+        for (int pl = 0; pl < 3; ++pl) *reinterpret_cast<bf16x8*>(o + pl * 1024) = p[pl];
     }
 }
 
@@ -2174,7 +2419,6 @@ const void* conv_q_kernel() {
 
 template <int CK, int KT>
 const void* conv_q_kernel_epi(int epi) {
-    if (epi == QEPI_ADAIN_BWD) return conv_q_kernel<CK, KT, QEPI_ADAIN_BWD>();
     if (epi == QEPI_STATS) return conv_q_kernel<CK, KT, QEPI_STATS>();
     return conv_q_kernel<CK, KT, QEPI_STORE>();
 }
@@ -2184,6 +2428,36 @@ const void* conv_q_kernel_for(int CK, int k, int epi) {
     if (k == 7 && CK == CGQ_CK7) return conv_q_kernel_epi<CGQ_CK7, 7>(epi);
     if (k == 11 && CK == CGQ_CK11) return conv_q_kernel_epi<CGQ_CK11, 11>(epi);
     return nullptr;
+}
+
+// LDS bytes of one split_gemm block: two stages of the input window's three
+// bf16 planes.
+size_t split_lds_bytes(int G, int d) { return 2 * 3 * static_cast<size_t>(BN + (G - 1) * d) * 32; }
+
+template <int KT, int EPI>
+const void* split_kernel() {
+    static bool attr = false;
+    if (!attr) {
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&split_gemm<KT, EPI>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        attr = true;
+    }
+    return reinterpret_cast<const void*>(&split_gemm<KT, EPI>);
+}
+
+template <int KT>
+const void* split_kernel_epi(int epi) {
+    if (epi == QEPI_ADAIN_BWD) return split_kernel<KT, QEPI_ADAIN_BWD>();
+    return split_kernel<KT, QEPI_STORE>();
+}
+
+// The instance with the tap loop unrolled where all k taps' window fits one
+// chunk (the decoder's 3, 7 and 11), else the one that loops.
+const void* split_kernel_for(int k, int G, int epi) {
+    if (G == k && k == 3) return split_kernel_epi<3>(epi);
+    if (G == k && k == 7) return split_kernel_epi<7>(epi);
+    if (G == k && k == 11) return split_kernel_epi<11>(epi);
+    return split_kernel_epi<0>(epi);
 }
 
 // Input channels per K chunk: a power of two in [2, 32] so that it divides
@@ -2283,7 +2557,19 @@ void choose_chunks(kdec_ctx* ctx, GemmArgs& g, int C, int kk, int dd, long tiles
     g.cin_pad = static_cast<int>(cdiv(C, 32) * 32);
 }
 
-// Launches conv_gemm over an already packed A.
+// K chunking of split_gemm for a stride-1 correlation of k taps at dilation d
+// over C channels: as many taps per chunk as the staged window takes.
+void split_setup(GemmArgs& g, int C, int k, int d) {
+    const long fit = (SPLIT_SPAN - BN) / d + 1L;
+    g.G = static_cast<int>(std::min(static_cast<long>(k), fit));
+    g.n_tg = static_cast<int>(cdiv(k, g.G));
+    g.n_c16 = static_cast<int>(cdiv(C, 16));
+}
+
+// Floats of split_gemm's weight panel for M output rows.
+long split_panel(const GemmArgs& g, int M) { return cdiv(M, BM) * g.n_c16 * g.k * SPLIT_STEP; }
+
+// Launches a GEMM kernel over an already packed A.
 //
 // Work plan: with S resident blocks, T tiles take T / S whole rounds plus a
 // last round of r = T mod S tiles. When r is well below S, the last r tiles
@@ -2293,30 +2579,34 @@ void choose_chunks(kdec_ctx* ctx, GemmArgs& g, int C, int kk, int dd, long tiles
 int run_gemm(kdec_ctx* ctx, GemmArgs g, int N, int m_tiles, const char* fam,
              double flops) {
     const int CK = g.CK;
-    const bool octet = g.G > 0;
+    const bool split = g.n_c16 > 0;
+    const bool octet = !split && g.G > 0;
     const int kk = g.n_phase > 1 ? g.ph_kt : g.k;
     const int ss = g.n_phase > 1 ? 1 : g.s;
     const int dd = g.n_phase > 1 ? 1 : g.d;
-    if (octet ? (ss != 1 || g.G > kk || g.span8 < BN + (g.G - 1) * dd || g.span8 % 16)
+    if (split ? (ss != 1 || g.G > kk || BN + static_cast<long>(g.G - 1) * dd > SPLIT_SPAN)
+        : octet ? (ss != 1 || g.G > kk || g.span8 < BN + (g.G - 1) * dd || g.span8 % 16)
               : (CK * kk > 64 || (CK * kk) % 2))
         return fail(ctx, KDEC_EINVAL, "conv: bad chunk geometry");
     const bool quad = g.quad != 0;
     const int epi = g.ad.part ? QEPI_ADAIN_BWD : g.fs.part ? QEPI_STATS : QEPI_STORE;
-    if (!quad && epi != QEPI_STORE) return fail(ctx, KDEC_EINVAL, "conv: fused epilogue needs the quad kernel");
+    if (epi == QEPI_ADAIN_BWD ? !split : epi == QEPI_STATS && !quad)
+        return fail(ctx, KDEC_EINVAL, "conv: no such epilogue in this kernel");
     if (quad && (octet || g.n_phase > 1 || g.s != 1 || !conv_q_kernel_for(CK, g.k, epi)))
         return fail(ctx, KDEC_EINVAL, "conv: bad quad geometry");
-    size_t lds = octet ? 2 * (static_cast<size_t>(g.G) * 1024 + 8 * static_cast<size_t>(g.span8)) * sizeof(float)
+    size_t lds = split ? split_lds_bytes(g.G, dd)
+               : octet ? 2 * (static_cast<size_t>(g.G) * 1024 + 8 * static_cast<size_t>(g.span8)) * sizeof(float)
                : quad ? quad_lds_bytes(CK, g.k, g.d)
                       : conv_lds_bytes(CK, kk, ss, dd);
     if (static_cast<long>(g.C_in) * g.L_in * 4 > 0x7fffffffL)
         return fail(ctx, KDEC_EINVAL, "conv: input too large for one buffer descriptor");
     g.ybuf = (static_cast<long>(g.C_out) + BM) * g.L_y * 4 < 0x7fffffffL ? 1 : 0;
-    const void* kern = octet ? corr_kernel() : quad ? conv_q_kernel_for(CK, g.k, epi) : conv_kernel_for(CK);
+    const void* kern = split ? split_kernel_for(kk, g.G, epi) : octet ? corr_kernel() : quad ? conv_q_kernel_for(CK, g.k, epi) : conv_kernel_for(CK);
     if (!kern) return fail(ctx, KDEC_EINVAL, "conv: unsupported channel chunk");
     // conv_gemm with one LDS stage where two leave at most two blocks per CU
     // and one leaves more (the long windows of large strides)
     g.single = 0;
-    if (!octet && !quad && blocks_per_cu(kern, lds) <= 2 && blocks_per_cu(kern, lds / 2) > blocks_per_cu(kern, lds)) {
+    if (!split && !octet && !quad && blocks_per_cu(kern, lds) <= 2 && blocks_per_cu(kern, lds / 2) > blocks_per_cu(kern, lds)) {
         g.single = 1;
         lds /= 2;
     }
@@ -2329,10 +2619,12 @@ int run_gemm(kdec_ctx* ctx, GemmArgs g, int N, int m_tiles, const char* fam,
     const long tiles = static_cast<long>(g.m_tiles) * g.q_tiles * g.nz;
     if (tiles > 0x7fffffffL / 16) return fail(ctx, KDEC_EINVAL, "conv: grid too large");
     const long slots = static_cast<long>(blocks_per_cu(kern, lds)) * ctx->num_cus;
-    const int nchunks = octet ? g.n_oct * g.n_tg : g.cin_pad / CK;
+    // a part keeps at least four chunks, of split_gemm at least eight steps (16 channels by one tap)
+    const long parts = split ? std::min(static_cast<long>(g.n_c16) * g.n_tg, static_cast<long>(g.n_c16) * kk / 8)
+                             : (octet ? g.n_oct * g.n_tg : g.cin_pad / CK) / 4;
     const long rem = tiles % slots;
     long f = 1;
-    if (rem > 0) f = std::min(std::min(slots / rem, static_cast<long>(nchunks / 4)), 16L);
+    if (rem > 0) f = std::min(std::min(slots / rem, parts), 16L);
     if (f < 2) f = 1;
     g.fsplit = static_cast<int>(f);
     g.split_tiles = f > 1 ? static_cast<int>(rem) : 0;
@@ -2432,7 +2724,7 @@ int conv_fwd_impl(kdec_ctx* ctx, const float* X, long x_bs, const float* W, cons
     KDEC_CHECK(ctx, tot <= 0x7fffffffL && static_cast<long>(C_out) * C_in * k <= 0x7fffffffL,
                "kdec_conv1d_fwd: weights too large");
     if (g.quad)
-        hipLaunchKernelGGL(pack_quad, dim3(grid1d(tot / 4)), dim3(256), 0, ctx->stream, W, A.as<float>(), 0, C_in,
+        hipLaunchKernelGGL(pack_quad, dim3(grid1d(tot / 4)), dim3(256), 0, ctx->stream, W, A.as<float>(), C_in,
                            C_out, k, g.CK, g.cin_pad / g.CK, nq, tot / 4);
     else if (g.G > 0)
         hipLaunchKernelGGL(pack_octet, dim3(grid1d(tot)), dim3(256), 0, ctx->stream, W, A.as<float>(), 0, C_in,
@@ -2522,17 +2814,14 @@ struct AdainBwdIn {
     const float* alpha;
 };
 
-// Whether an input-grad GEMM of this geometry runs conv_gemm_q (whose
-// epilogue, and tile_reduce_adain's, can apply an AdaIN backward).
-bool dgrad_is_quad(kdec_ctx* ctx, int N, int C_in, int L, int C_out, int k, int dil) {
-    if (pick_ck_q(k) <= 0) return false;
-    GemmArgs g{};
-    choose_chunks(ctx, g, C_out, k, dil, cdiv(C_in, BM) * cdiv(L, BN) * N);
-    return g.G == 0;
+// Whether an input grad of this many output tiles applies an AdaIN backward
+// in its epilogue: four tiles per CU.
+bool dgrad_fuses(kdec_ctx* ctx, int N, int C_in, int L) {
+    return cdiv(C_in, BM) * cdiv(L, BN) * N >= 4L * ctx->num_cus;
 }
 
 // The input grad as a correlation of dY with the flipped weights; with `ad`
-// (only where dgrad_is_quad) dX receives ds = dX * act'(s) of that AdaIN and
+// (beta = 0) dX receives ds = dX * act'(s) of that AdaIN and
 // `part` its row partial sums (2 * q_tiles slots per row).
 int conv_dgrad_impl(kdec_ctx* ctx, const float* W, const float* dY, long dy_bs, float* dX, long dx_bs, int N,
                     int C_in, int L, int C_out, int k, int stride, int pad, int dil, float scale, float beta,
@@ -2554,13 +2843,9 @@ int conv_dgrad_impl(kdec_ctx* ctx, const float* W, const float* dY, long dy_bs, 
     g.m_pad = m_pad;
     g.k = k; g.s = 1; g.d = dil; g.p = pp; g.n_q = L;
     g.scale = scale; g.beta = beta; g.n_phase = 1;
-    choose_chunks(ctx, g, C_out, k, dil, cdiv(C_in, BM) * cdiv(L, BN) * N);
-    if (g.G == 0 && pick_ck_q(k) > 0) {
-        g.quad = 1;
-        g.CK = pick_ck_q(k);
-    }
+    split_setup(g, C_out, k, dil);
     if (ad) {
-        if (!g.quad || beta != 0.0f) return fail(ctx, KDEC_EINVAL, "conv dgrad: no AdaIN epilogue for this geometry");
+        if (beta != 0.0f) return fail(ctx, KDEC_EINVAL, "conv dgrad: no AdaIN epilogue for this geometry");
         g.ad.x = ad->X;
         g.ad.x_bs = ad->x_bs;
         g.ad.st = reinterpret_cast<const float2*>(ad->stats);
@@ -2573,29 +2858,15 @@ int conv_dgrad_impl(kdec_ctx* ctx, const float* W, const float* dY, long dy_bs, 
         g.ad.part = part;
         g.ad.nch = nch;
     }
-    const int nq = static_cast<int>(cdiv(static_cast<long>(g.CK) * k / 2, 4));
-    const long tot = g.quad ? (m_pad / BM) * static_cast<long>(g.cin_pad / g.CK) * nq * 1024
-                            : static_cast<long>(g.cin_pad) * k * m_pad;
+    const long tot = split_panel(g, C_in);
     Workspace A(ctx, static_cast<size_t>(tot) * sizeof(float));
     if (!A.p) return KDEC_ENOMEM;
     g.A = A.as<float>();
     KDEC_CHECK(ctx, tot <= 0x7fffffffL && static_cast<long>(C_out) * C_in * k <= 0x7fffffffL,
                "kdec_conv1d_dgrad: weights too large");
-    if (g.quad)
-        hipLaunchKernelGGL(pack_quad, dim3(grid1d(tot / 4)), dim3(256), 0, ctx->stream, W, A.as<float>(), 1, C_in,
-                           C_out, k, g.CK, g.cin_pad / g.CK, nq, tot / 4);
-    else if (g.G > 0)
-        hipLaunchKernelGGL(pack_octet, dim3(grid1d(tot)), dim3(256), 0, ctx->stream, W, A.as<float>(), 1, C_in,
-                           C_out, k, 1, k, m_pad, static_cast<int>(tot), 1);
-    else
-        if (g.cin_pad % g.CK == 0 && m_pad % 64 == 0 && k <= 32)
-            hipLaunchKernelGGL(pack_dgrad_t, dim3(static_cast<unsigned>(cdiv(g.cin_pad, 4)),
-                                                  static_cast<unsigned>(m_pad / 64)),
-                               dim3(256), 4 * 64 * k * sizeof(float), ctx->stream, W, A.as<float>(), C_in, C_out, k,
-                               g.cin_pad, m_pad, g.CK);
-        else
-            hipLaunchKernelGGL(pack_dgrad, dim3(grid1d(tot)), dim3(256), 0, ctx->stream, W, A.as<float>(), C_in,
-                               C_out, k, g.cin_pad, m_pad, g.CK);
+    const long items = tot / SPLIT_STEP * 256;
+    hipLaunchKernelGGL(pack_split, dim3(grid1d(items)), dim3(256), 0, ctx->stream, W, A.as<float>(), C_in, C_out, k,
+                       g.n_c16 * k, items);
     if (int rc = launch_check(ctx, "pack_dgrad")) return rc;
     return run_gemm(ctx, g, N, m_pad / BM, "conv_dgrad",
                     2.0 * N * C_out * static_cast<double>(L_out) * C_in * k);
@@ -2630,11 +2901,11 @@ int kdec_conv1d_dgrad_adain_bwd(kdec_ctx* ctx, const float* W, const float* dY, 
     KDEC_CHECK(ctx, x_bs >= static_cast<long>(C_in) * L && dx_bs >= static_cast<long>(C_in) * L &&
                         (!R || r_bs >= static_cast<long>(C_in) * L),
                "kdec_conv1d_dgrad_adain_bwd: batch stride too small");
-    // fused where the input grad runs conv_gemm_q and dX aliases neither the
+    // fused where the grid is large enough and dX aliases neither the
     // AdaIN input nor R (ds is staged in dX); else the two calls it replaces
     const bool fuse = stride == 1 && dX != X && dX != R &&
                       (static_cast<long>(C_in) + BM) * L * 4 < 0x7fffffffL &&
-                      dgrad_is_quad(ctx, N, C_in, L, C_out, k, dil);
+                      dgrad_fuses(ctx, N, C_in, L);
     if (!fuse) {
         Workspace t(ctx, static_cast<size_t>(N) * C_in * L * sizeof(float));
         if (!t.p) return KDEC_ENOMEM;
@@ -2893,7 +3164,7 @@ int convt_fwd_impl(kdec_ctx* ctx, const float* X, long x_bs, const float* W, con
     KDEC_CHECK(ctx, ph * stride <= 0x7fffffffL && static_cast<long>(C_out) * C_in * k <= 0x7fffffffL,
                "kdec_convt1d_fwd: weights too large");
     if (g.G > 0)
-        hipLaunchKernelGGL(pack_octet, dim3(grid1d(ph * stride)), dim3(256), 0, ctx->stream, W, A.as<float>(), 2,
+        hipLaunchKernelGGL(pack_octet, dim3(grid1d(ph * stride)), dim3(256), 0, ctx->stream, W, A.as<float>(), 1,
                            C_in, C_out, k, stride, kt, m_pad, static_cast<int>(ph), stride);
     else
         hipLaunchKernelGGL(pack_convt_fwd, dim3(grid1d(ph * stride)), dim3(256), 0, ctx->stream, W,
