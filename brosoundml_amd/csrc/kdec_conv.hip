@@ -28,9 +28,10 @@
 // the kernel at ~80 VGPRs and 4-6 waves per SIMD.
 //
 // Weight-grad (`wgrad_gemm`): dW[m, (c, t)] = sum_{n, l} dY[n, m, l] *
-// X[n, c, l*s + t*d - p], a GEMM with the huge position axis as K. It is
-// split over K into deterministic partial tiles that a second kernel sums in
-// a fixed order; the bias grad (row sums of dY) rides along in the same pass.
+// X[n, c, l*s + t*d - p], a GEMM with the huge position axis as K, on split
+// bf16 terms like split_gemm. It is split over K into deterministic partial
+// tiles that a second kernel sums in a fixed order; the bias grad (row sums of
+// dY) rides along in the same pass.
 #include "kdec_buffer.hpp"
 #include "kdec_internal.hpp"
 #include "kdec_snake_math.hpp"
@@ -1180,6 +1181,26 @@ __device__ inline void split_mma(const bf16x8 (&a)[3][2], const bf16x8 (&b)[3][2
 #undef KDEC_SPLIT_MMA
 }
 
+// The two accumulators' sum into hh; true where the wave has to form its sums
+// again on the float unit from the unsplit operands. An infinity splits as
+// inf + NaN + NaN, a float above the largest bf16 likewise, and the matrix
+// unit reads subnormal bf16 as zero, so the lower terms of operands under
+// 2^-110 are lost: a wave with a column that is not finite, or not zero yet
+// under 2^-90, goes back, and such inputs give what they give there.
+__device__ inline bool split_finish(f32x16 (&hh)[2][2], const f32x16 (&lo)[2][2], bool live) {
+    float mag = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                hh[i][j][e] += lo[i][j][e];
+                mag += fabsf(hh[i][j][e]);
+            }
+    return live && __any(!(mag <= 3.4028235e38f) || (mag > 0.0f && mag < 0x1p-90f));
+}
+
 template <int KT, int EPI>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2)))
 void split_gemm(GemmArgs g) {
@@ -1314,27 +1335,7 @@ void split_gemm(GemmArgs g) {
         if (ch + 1 < ch1) store_x(buf ^ 1);
         __syncthreads();
     }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] += lo[i][j][e];
-
-    // An infinity splits as inf + NaN + NaN, a float above the largest bf16
-    // likewise, and the matrix unit reads subnormal bf16 as zero, so the lower
-    // terms of operands under 2^-110 are lost. A wave with a column that is
-    // not finite, or not zero yet under 2^-90, forms its sums again on the
-    // float unit from the unsplit operands: such inputs give what they give
-    // there.
-    float mag = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) mag += fabsf(acc[i][j][e]);
-    if (live && __any(!(mag <= 3.4028235e38f) || (mag > 0.0f && mag < 0x1p-90f))) {
+    if (split_finish(acc, lo, live)) {
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -1848,49 +1849,84 @@ __global__ void pack_split(const float* W, float* A, int C_in, int C_out, int k,
 
 // ─── weight grad ─────────────────────────────────────────────────────────
 
-constexpr int KC = 32;       // positions per K chunk
-// Waves along n (2 along m): 4 (256 columns per block) or 2 (128 columns,
-// for column counts C_x * k that 256-wide tiles would leave partly idle).
-constexpr int WG_WN = 4;
-constexpr int WG_NT = 128 * WG_WN;       // threads per wide wgrad block
-constexpr int WG_BN = 64 * WG_WN;        // n columns per wide wgrad block
-// G tile in LDS: 64 row pairs (m, m + 64) of 2*KC positions at a pair stride
-// of 2*KC + 4 floats: one 64-lane load fills a whole pair, rows stay 16-B
-// aligned for ds_read_b128, and 16 consecutive m of one such read cover all
-// 64 banks once.
-constexpr int GP = 2 * KC + 4;
-// Held packed input-window offsets per wave on the stride-1 fast path.
-constexpr int WG_XI = 8;
+constexpr int KC = 32;        // positions per K chunk
+constexpr int WG_BN = 128;    // columns per block: four 32-column blocks
+constexpr int WG_GO = 2048 + 32;    // bytes of one octet of positions over the 128 G rows (padded: see wgrad_gemm)
+constexpr int WG_GPL = 4 * WG_GO;   // bytes of one G plane
 
 struct WgradArgs {
     const float* X;      // correlation input  [n][C_x][L_x]
     long x_bs;
     const float* G;      // grad rows (A side) [n][M][L_g]
     long g_bs;
-    float* P;            // partials [split][M][NN]
+    float* P;            // partials [split][cdiv(M, 4)][n_tiles * 128][4]
     float* Pb;           // bias partials [split][M] (sum of G), or null
-    int M, C_x, L_x, L_g, k, s, d, p;
-    int NN;              // C_x * k
+    int M, C_x, L_x, L_g, k, s, p;
+    // Column (c, t) as virtual channel v = c * R + r and tap q, t = q * R + r:
+    // at position l it meets X[c][(l + q * sh) * s + r * rd - p].
+    //   stride 1          R = 1, T = k, sh = d
+    //   strided, d = 1    R = s, rd = 1, T = cdiv(k, s), sh = 1
+    //   strided, dilated  R = k, rd = d, T = 1
+    int R, rd, T, sh;
+    int NB;              // 32-column blocks: cdiv(C_x * R, 32) channel groups x T taps, tap fastest
     int chunks_per_n, total_chunks, splits;
     int n_tiles, m_tiles;
-    int XR;              // staged input rows per n-tile
-    int span, segs;      // input-row staging: `span` positions as segs loads of up to 64
-    int rs;              // LDS row stride of the staged input rows
-    int blk4;            // P in row quads: [split][M / 4][NN][4] (M a multiple of 4)
+    int rows;            // LDS rows of the input stage (the most any column tile needs)
 };
 
-// P[z, m, c*k + t] = sum over this split's positions l of
-//   G[n, m, l] * X[n, c, l*s + t*d - p]
-// (and Pb[z, m] = sum of G over the same positions, from the n-tile-0 blocks).
-// 1-D grid of n_tiles * m_tiles * splits blocks. Both operands run along the
-// position axis in memory, so they are staged row by row straight into LDS
-// (buffer_load_dword ... lds, zero past each row's end): G as 128 rows of KC
-// positions at an odd row stride, the input window as XR channel rows at a
-// stride rs chosen so that column n = c*k + t lands on bank n*d.
-template <bool S1, int WN>  // S1: stride 1 (the four input values of a group are adjacent)
-__global__ __launch_bounds__(128 * WN) __attribute__((amdgpu_waves_per_eu(4)))
+// Where the four column blocks of tile nt read the staged input: consecutive
+// taps of one channel group share a window of KC + (taps - 1) * sh positions
+// (one tap each where the taps lie further apart than a chunk).
+struct WgradCols {
+    int cg[4], q[4];  // channel group, tap (cg < 0: past the last block)
+    int seg[4];       // first LDS row of the block's segment (-1: continues the one before)
+    int row[4];       // LDS row of position 0 at its tap
+    int rows;
+};
+
+__host__ __device__ inline WgradCols wgrad_cols(int nt, int NB, int T, int sh) {
+    WgradCols w;
+    w.rows = 0;
+    int seg0 = 0, q0 = 0;
+    for (int j = 0; j < 4; ++j) {
+        const int nb = nt * 4 + j;
+        const int cg = nb / T, q = nb - cg * T;
+        const bool in = nb < NB;
+        const bool join = in && j > 0 && q > 0 && sh <= KC;  // the block before is tap q - 1 of the same group
+        if (in && !join) {
+            seg0 = w.rows;
+            q0 = q;
+        }
+        w.cg[j] = in ? cg : -1;
+        w.q[j] = q;
+        w.seg[j] = in && !join ? seg0 : -1;
+        w.row[j] = in ? seg0 + (q - q0) * sh : 0;
+        if (in) w.rows = seg0 + (q - q0) * sh + KC;
+    }
+    return w;
+}
+
+// P[z, m, column] = sum over this split's positions l of G[n, m, l] *
+// X[n, c, (l + q sh) s + r rd - p] (and Pb[z, m] = sum of G over the same
+// positions, from the column-tile-0 blocks), on split bf16 terms as
+// split_gemm; positions are the K axis. Bound: MFMA, then the splitting of G
+// (once per 128 columns). 1-D grid of n_tiles * m_tiles * splits blocks of a
+// 128 x 128 tile (2 x 2 waves of 64 x 64).
+//
+// A chunk is KC positions. G goes to LDS as [octet of positions][row][8]
+// (loaded 32 bytes per lane along the row; the octets 2080 bytes apart, so
+// that both the stores, four octets by two rows at a time, and the 16-byte
+// fragment reads, 32 rows of one octet, spread over the banks), X
+// channels-last as [position][32 channels]. A tap is then a shift by whole
+// 64-byte rows, and the fragment of eight consecutive positions of a column
+// is two transposing reads (ds_read_b64_tr_b16: 16 lanes read four rows of 16
+// channels, lane i receives the four positions of channel i). Both operands
+// are loaded to registers while the previous chunk is multiplied.
+template <bool S1>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2)))
 void wgrad_gemm(WgradArgs g) {
     extern __shared__ float smem[];
+    char* lds = reinterpret_cast<char*>(smem);
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1903,235 +1939,236 @@ void wgrad_gemm(WgradArgs g) {
     const int mt = lid % g.m_tiles;
     const int z = lid / g.m_tiles;
     const int m0 = mt * BM;
-    const int n0 = nt * (64 * WN);
-    const int k = g.k, s = S1 ? 1 : g.s, d = g.d;
-    const int ci_lo = n0 / k;
-    const int gsz = 64 * GP;
-    const int stage = gsz + (g.XR * g.rs + 63) / 64 * 64;  // as wgrad_layout
     const bool do_bias = g.Pb && nt == 0;
-    // a wave whose 64 columns all lie past NN (the last n-tile) only stages
-    const bool live = n0 + wn * 64 < g.NN;
-    constexpr unsigned OOB = 0x80000000u;  // any offset >= the buffer size reads 0
+    const WgradCols cols = wgrad_cols(nt, g.NB, g.T, g.sh);
+    // this wave's two column blocks
+    const int cgw[2] = {wn ? cols.cg[2] : cols.cg[0], wn ? cols.cg[3] : cols.cg[1]};
+    const int qw[2] = {wn ? cols.q[2] : cols.q[0], wn ? cols.q[3] : cols.q[1]};
+    const bool live = cgw[0] >= 0;  // wave-uniform (the blocks past the last come last)
+    const int s = S1 ? 1 : g.s, R = S1 ? 1 : g.R;
+    const int xpl = g.rows * 64;                    // bytes of one X plane
+    const int stage = 3 * WG_GPL + 3 * xpl;
+    constexpr unsigned OOB = 0x80000000u;           // any offset past the buffer reads 0
 
-    // this lane's two B columns: staged row offset of (c - ci_lo, t)
-    int xcol[2];
+    // G items: rows wave * 16 + lane / 4 and 64 on, octet lane % 4.
+    const int g_oct = lane & 3, g_row = wave * 16 + (lane >> 2);
+    // X items e = tid, tid + 256: LDS row e / 4, channels 8 (e % 4) .. + 7 of
+    // the row's group; its position offset and first virtual channel
+    int x_u[2], x_v[2];
+    bool x_in[2];
 #pragma unroll
-    for (int tn = 0; tn < 2; ++tn) {
-        const int n = n0 + wn * 64 + tn * 32 + l32;
-        const int c = n / k;
-        xcol[tn] = (c - ci_lo) * g.rs + (n - c * k) * d;
+    for (int i = 0; i < 2; ++i) {
+        const int e = tid + i * NT, row = e >> 2;
+        x_in[i] = row < cols.rows;
+        x_u[i] = 0;
+        x_v[i] = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (cols.seg[j] >= 0 && row >= cols.seg[j]) {
+                x_u[i] = row - cols.seg[j] + cols.q[j] * g.sh;
+                x_v[i] = cols.cg[j] * 32 + (e & 3) * 8;
+            }
     }
-    const int g_row_lane = lane >> 5;      // 0: row m0 + i, 1: row m0 + i + 64
-    const int g_pos_lane = lane & 31;
+    const bool two = wave * 64 + NT < 4 * cols.rows;  // wave-uniform
 
-    // One buffer descriptor per utterance; rows, positions and channels out
-    // of range get an out-of-bounds offset and stage as zeros. Wave w stages
-    // G row pairs w, w + 8, ... and input rows w, w + 8, ... (all segments of
-    // each), with the range checks skipped for chunks wholly inside.
-    // Fast staging plan for chunks wholly inside their rows: per-lane byte
-    // offsets at chunk position 0, fixed for the block, with the chunk's start
-    // in the scalar offset, so one DMA costs one M0 write and the load. The
-    // input window is staged packed: instruction j fills LDS floats
-    // [64j, 64j + 64) of the [row][rs] window, lanes past a row's span (and
-    // rows past C_x) read out of range and stage zeros.
-    constexpr int GI = 64 / (2 * WN);  // G pair rows per wave
-    const bool g_rows_in = m0 + BM <= g.M;  // uniform: whole m-tile (else the checked path)
-    // pair row wave + 8j of this lane: g_off + j * 8 * L_g * 4
-    const unsigned g_off = static_cast<unsigned>((m0 + wave + 64 * g_row_lane) * g.L_g + g_pos_lane) * 4u;
-    const int g_step = 2 * WN * g.L_g * 4;
-    // Stride 1: the wave's packed-instruction offsets are held (windows of up
-    // to WG_XI * 8 * 64 floats; larger ones take the checked path). Strided:
-    // this lane's slot of the wave's first instruction as (row, position),
-    // each further instruction of the wave 8 * 64 slots on.
-    const int nxi = (g.XR * g.rs + 63) / 64;  // packed-window instructions
-    const bool fast_x = !S1 || nxi <= WG_XI * 2 * WN;  // uniform per launch
-    unsigned x_off[S1 ? WG_XI : 1];
-    if (S1) {
+    float gr[2][8], xr[2][8];
+    auto load_x_item = [&](int i, const __amdgpu_buffer_rsrc_t& xrs, int l0) {
+        if constexpr (S1) {
+            const int pos = l0 + x_u[i] - g.p;
+            unsigned off = x_in[i] && pos >= 0 && pos < g.L_x
+                               ? static_cast<unsigned>(x_v[i] * g.L_x + pos) * 4u : OOB;
 #pragma unroll
-        for (int j = 0; j < WG_XI; ++j) {
-            const int slot = (wave + 2 * WN * j) * 64 + lane;
-            const int r = slot / g.rs, pos = slot - r * g.rs;
-            const int c = ci_lo + r;
-            x_off[S1 ? j : 0] = (r < g.XR && pos < g.span && c < g.C_x)
-                                    ? static_cast<unsigned>(c * g.L_x + pos) * 4u : OOB;
+            for (int j = 0; j < 8; ++j) {
+                xr[i][j] =
+                    __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrs, static_cast<int>(off), 0, 0));
+                off += g.L_x * 4;
+            }
+        } else {
+            int c = x_v[i] / R, r = x_v[i] - c * R;
+            const int pos0 = (l0 + x_u[i]) * s - g.p;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int pos = pos0 + r * g.rd;
+                const unsigned off =
+                    x_in[i] && pos >= 0 && pos < g.L_x ? static_cast<unsigned>(c * g.L_x + pos) * 4u : OOB;
+                xr[i][j] =
+                    __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrs, static_cast<int>(off), 0, 0));
+                if (++r == R) {
+                    r = 0;
+                    ++c;
+                }
+            }
         }
-    }
-    const int xs0 = wave * 64 + lane;
-    const int xr0 = xs0 / g.rs, xp0 = xs0 - xr0 * g.rs;
-    const int xqd = (2 * WN * 64) / g.rs, xrd = (2 * WN * 64) - xqd * g.rs;
-    auto issue = [&](int ch, int sb) {
+    };
+    auto load = [&](int ch) {
         const int b = ch / g.chunks_per_n;
         const int l0 = (ch - b * g.chunks_per_n) * KC;
         const __amdgpu_buffer_rsrc_t grs = uniform_rsrc(g.G + static_cast<long>(b) * g.g_bs, g.M * g.L_g * 4);
         const __amdgpu_buffer_rsrc_t xrs = uniform_rsrc(g.X + static_cast<long>(b) * g.x_bs, g.C_x * g.L_x * 4);
-        const int x0 = l0 * s - g.p;
-        if (S1 && fast_x && x0 >= 0 && x0 + g.span <= g.L_x) {  // uniform
+        const int l = l0 + g_oct * 8;
 #pragma unroll
-            for (int j = 0; j < WG_XI; ++j)
-                if (wave + 2 * WN * j < nxi)
-                    __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, smem + sb + gsz + (wave + 2 * WN * j) * 64, 4,
-                                                             static_cast<int>(x_off[S1 ? j : 0]), x0 * 4, 0, 0);
-        } else if (!S1 && x0 >= 0 && x0 + g.span <= g.L_x) {  // uniform
-            int r = xr0, pp = xp0;
-            for (int jj = wave; jj < nxi; jj += 2 * WN) {
-                const int c = ci_lo + r;
-                const unsigned off = (r < g.XR && pp < g.span && c < g.C_x)
-                                         ? static_cast<unsigned>(c * g.L_x + pp) * 4u : OOB;
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, smem + sb + gsz + jj * 64, 4, static_cast<int>(off),
-                                                         x0 * 4, 0, 0);
-                pp += xrd;
-                r += xqd;
-                if (pp >= g.rs) {
-                    pp -= g.rs;
-                    ++r;
+        for (int i = 0; i < 2; ++i) {
+            const unsigned off = static_cast<unsigned>((m0 + g_row + 64 * i) * g.L_g + l) * 4u;
+            if (l0 + KC <= g.L_g) {  // uniform
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const u32x4 v = __builtin_bit_cast(
+                        u32x4, __builtin_amdgcn_raw_buffer_load_b128(grs, static_cast<int>(off + 16 * h), 0, 0));
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) gr[i][4 * h + j] = __uint_as_float(v[j]);
                 }
-            }
-        } else {
-            const bool x_in = x0 >= 0 && x0 + g.span <= g.L_x;  // uniform
-            for (int r = wave; r < g.XR; r += 2 * WN) {
-                const int c = ci_lo + r;
-                const bool c_in = c < g.C_x;  // uniform
-                int pos = x0 + lane;
-                for (int sg = 0; sg < g.segs; ++sg, pos += 64) {
-                    const unsigned off = (c_in && (x_in || (pos >= 0 && pos < g.L_x)))
-                                             ? static_cast<unsigned>(c * g.L_x + pos) * 4u : OOB;
-                    if (sg * 64 + lane < g.span)  // exactly the row's span: rows pack at stride rs >= span
-                        __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, smem + sb + gsz + r * g.rs + sg * 64, 4,
-                                                                 static_cast<int>(off), 0, 0, 0);
-                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    gr[i][j] = __builtin_bit_cast(
+                        float, __builtin_amdgcn_raw_buffer_load_b32(
+                                   grs, static_cast<int>(l + j < g.L_g ? off + 4 * j : OOB), 0, 0));
             }
         }
-        if (g_rows_in && l0 + KC <= g.L_g) {  // uniform
-            // the row step rides in the scalar offset: one lane offset for all
+        load_x_item(0, xrs, l0);
+        if (two) load_x_item(1, xrs, l0);
+    };
+    double bsum[2] = {0.0, 0.0};
+    auto store8 = [&](const float (&v)[8], char* p, int plane) {
+        bf16x8 h, m, l;
 #pragma unroll
-            for (int j = 0; j < GI; ++j)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(grs, smem + sb + (wave + 2 * WN * j) * GP, 4,
-                                                         static_cast<int>(g_off), l0 * 4 + j * g_step, 0, 0);
-            return;
+        for (int j = 0; j < 8; ++j) {
+            __bf16 a, b, c;
+            split3(v[j], a, b, c);
+            h[j] = a;
+            m[j] = b;
+            l[j] = c;
         }
-        const int l = l0 + g_pos_lane;  // a partial m-tile or the last chunk of a row: checked
-        for (int i = wave; i < 64; i += 2 * WN) {
-            const int m = m0 + i + 64 * g_row_lane;
-            const unsigned off = (m < g.M && l < g.L_g) ? static_cast<unsigned>(m * g.L_g + l) * 4u : OOB;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(grs, smem + sb + i * GP, 4, static_cast<int>(off), 0, 0, 0);
+        *reinterpret_cast<bf16x8*>(p) = h;
+        *reinterpret_cast<bf16x8*>(p + plane) = m;
+        *reinterpret_cast<bf16x8*>(p + 2 * plane) = l;
+    };
+    auto store = [&](int buf) {
+        char* st = lds + buf * stage;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            if (do_bias)
+                bsum[i] += ((gr[i][0] + gr[i][1]) + (gr[i][2] + gr[i][3])) + ((gr[i][4] + gr[i][5]) + (gr[i][6] + gr[i][7]));
+            store8(gr[i], st + g_oct * WG_GO + (g_row + 64 * i) * 16, WG_GPL);
         }
+        if (x_in[0]) store8(xr[0], st + 3 * WG_GPL + tid * 16, xpl);
+        if (two && x_in[1]) store8(xr[1], st + 3 * WG_GPL + (tid + NT) * 16, xpl);
     };
 
-    f32x16 acc[2][2];
+    f32x16 acc[2][2], lo[2][2];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-    double bsum = 0.0;
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = lo[i][j][e] = 0.0f;
 
+    // fragment addresses within a stage: A row wm * 64 + l32 of octet hi; B
+    // position 8 hi + (lane & 15) / 4, channels 16 (lane / 16 & 1) + 4 (lane & 3) .. + 3
+    const int a_rd = hi * WG_GO + (wm * 64 + l32) * 16;
+    const int b_ln = (hi * 8 + ((lane & 15) >> 2)) * 64 + ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
+    const int b_rd0 = 3 * WG_GPL + (wn ? cols.row[2] : cols.row[0]) * 64 + b_ln;
+    const int b_rd1 = 3 * WG_GPL + (wn ? cols.row[3] : cols.row[1]) * 64 + b_ln;
     // split z: chunks [z * total / splits, (z + 1) * total / splits)
     const int ch0 = static_cast<int>(static_cast<long>(z) * g.total_chunks / g.splits);
     const int ch1 = static_cast<int>(static_cast<long>(z + 1) * g.total_chunks / g.splits);
-    if (ch0 < ch1) issue(ch0, 0);
-    __builtin_amdgcn_s_waitcnt(0);
+    if (ch0 < ch1) {
+        load(ch0);
+        store(0);
+    }
     __syncthreads();
     for (int ch = ch0; ch < ch1; ++ch) {
-        const int sb = ((ch - ch0) & 1) * stage;
-        __builtin_amdgcn_s_setprio(1);  // as in conv_gemm_q
-        if (ch + 1 < ch1) issue(ch + 1, stage - sb);
-        __builtin_amdgcn_s_setprio(0);
-        if (do_bias && tid < BM) {
-            float t = 0.0f;
-            const int row = sb + (tid & 63) * GP + (tid >> 6) * KC;
-            for (int kc = 0; kc < KC; ++kc) t += smem[row + kc];
-            bsum += t;
-        }
-        // group gi covers positions l0 + 8*gi + 4*h + e (e = 0..3) for lanes of
-        // half h: one ds_read_b128 per A row, four adjacent (stride s) input
-        // values per B column, then 16 MFMAs
-        const int ga = sb + l32 * GP + wm * KC + hi * 4;
-        const int xa0 = sb + gsz + xcol[0] + hi * 4 * s;
-        const int xa1 = sb + gsz + xcol[1] + hi * 4 * s;
-        auto ld = [&](int gi, float4 (&a)[2], float (&bv)[2][4]) {
-            gi = min(gi, KC / 8 - 1);
-            int go = ga + gi * 8;
-            int xo0 = xa0 + gi * 8 * s;
-            int xo1 = xa1 + gi * 8 * s;
-            asm volatile("" : "+v"(go), "+v"(xo0), "+v"(xo1));
-            a[0] = *reinterpret_cast<const float4*>(smem + go);
-            a[1] = *reinterpret_cast<const float4*>(smem + go + 32 * GP);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                bv[0][e] = smem[xo0 + e * s];
-                bv[1][e] = smem[xo1 + e * s];
-            }
-        };
-        auto mm = [&](const float4 (&a)[2], const float (&bv)[2][4]) {
-            const float a0[4] = {a[0].x, a[0].y, a[0].z, a[0].w};
-            const float a1[4] = {a[1].x, a[1].y, a[1].z, a[1].w};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[e], bv[0][e], acc[0][0], 0, 0, 0);
-                acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[e], bv[1][e], acc[0][1], 0, 0, 0);
-                acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[e], bv[0][e], acc[1][0], 0, 0, 0);
-                acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[e], bv[1][e], acc[1][1], 0, 0, 0);
-            }
-        };
+        const int buf = (ch - ch0) & 1;
+        if (ch + 1 < ch1) load(ch + 1);
         if (live) {
-            constexpr int NR = S1 ? 6 : 10;  // LDS reads per group
-            float4 pa[2], qa[2];
-            float pb[2][4], qb[2][4];
-            ld(0, pa, pb);
+            const char* st = lds + buf * stage;
 #pragma unroll
-            for (int gi = 0; gi < KC / 8; gi += 2) {
-                ld(gi + 1, qa, qb);
-                mm(pa, pb);
-                ld(gi + 2, pa, pb);
-                mm(qa, qb);
-                // (1 MFMA, 1 read) x NR, then the group's other MFMAs; twice
-                for (int r = 0; r < 2; ++r) {
-                    for (int i = 0; i < NR; ++i) {
-                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            for (int ks = 0; ks < KC / 16; ++ks) {
+                bf16x8 a[3][2], b[3][2];
+#pragma unroll
+                for (int pl = 0; pl < 3; ++pl)
+#pragma unroll
+                    for (int tm = 0; tm < 2; ++tm)
+                        a[pl][tm] = *reinterpret_cast<const bf16x8*>(st + pl * WG_GPL + 2 * ks * WG_GO + a_rd + tm * 512);
+#pragma unroll
+                for (int pl = 0; pl < 3; ++pl)
+#pragma unroll
+                    for (int tn = 0; tn < 2; ++tn) {
+                        typedef short s16x4 __attribute__((ext_vector_type(4)));
+                        typedef __attribute__((address_space(3))) s16x4* LdsP;
+                        const char* p = st + pl * xpl + ks * 1024 + (tn ? b_rd1 : b_rd0);
+                        const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsP)(p));
+                        const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsP)(p + 256));
+                        b[pl][tn] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
                     }
-                    __builtin_amdgcn_sched_group_barrier(0x008, 16 - NR, 0);
-                }
+                split_mma(a, b, acc, lo);
             }
         }
-        __builtin_amdgcn_s_waitcnt(0);  // this wave's staging loads landed
+        if (ch + 1 < ch1) store(buf ^ 1);
         __syncthreads();
     }
-
-    float* Pz = g.P + static_cast<long>(z) * g.M * g.NN;
-    if (g.blk4) {  // uniform: a lane's four consecutive rows of a column as one 16-byte store
+    if (split_finish(acc, lo, live)) {  // formed again on the float unit, two positions a step
 #pragma unroll
-        for (int tn = 0; tn < 2; ++tn) {
-            const int n = n0 + wn * 64 + tn * 32 + l32;
-            if (n >= g.NN) continue;
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int tm = 0; tm < 2; ++tm)
+            for (int j = 0; j < 2; ++j)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int m = m0 + wm * 64 + tm * 32 + 8 * j + 4 * hi;  // a multiple of 4
-                    if (m < g.M)
-                        reinterpret_cast<float4*>(Pz)[static_cast<long>(m >> 2) * g.NN + n] =
-                            make_float4(acc[tm][tn][4 * j], acc[tm][tn][4 * j + 1], acc[tm][tn][4 * j + 2],
-                                        acc[tm][tn][4 * j + 3]);
+                for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+        for (int ch = ch0; ch < ch1; ++ch) {
+            const int bt = ch / g.chunks_per_n;
+            const int l0 = (ch - bt * g.chunks_per_n) * KC;
+            const __amdgpu_buffer_rsrc_t grs = uniform_rsrc(g.G + static_cast<long>(bt) * g.g_bs, g.M * g.L_g * 4);
+            const __amdgpu_buffer_rsrc_t xrs = uniform_rsrc(g.X + static_cast<long>(bt) * g.x_bs, g.C_x * g.L_x * 4);
+            for (int l = l0 + hi; l < l0 + KC; l += 2) {
+                float av[2], bv[2];
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const int m = m0 + wm * 64 + u * 32 + l32;
+                    const unsigned ao = m < g.M && l < g.L_g ? static_cast<unsigned>(m * g.L_g + l) * 4u : OOB;
+                    av[u] = __builtin_bit_cast(float,
+                                               __builtin_amdgcn_raw_buffer_load_b32(grs, static_cast<int>(ao), 0, 0));
+                    const int v = cgw[u] * 32 + l32, c = v / R, r = v - c * R;
+                    const int pos = (l + qw[u] * g.sh) * s + (S1 ? 0 : r * g.rd) - g.p;
+                    const unsigned bo = v >= 0 && c < g.C_x && l < g.L_g && pos >= 0 && pos < g.L_x
+                                            ? static_cast<unsigned>(c * g.L_x + pos) * 4u : OOB;
+                    bv[u] = __builtin_bit_cast(float,
+                                               __builtin_amdgcn_raw_buffer_load_b32(xrs, static_cast<int>(bo), 0, 0));
                 }
-        }
-    } else {
 #pragma unroll
-        for (int tn = 0; tn < 2; ++tn) {
-            const int n = n0 + wn * 64 + tn * 32 + l32;
-            if (n >= g.NN) continue;
+                for (int tm = 0; tm < 2; ++tm)
 #pragma unroll
-            for (int tm = 0; tm < 2; ++tm)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    const int m = m0 + wm * 64 + tm * 32 + 8 * (e >> 2) + 4 * hi + (e & 3);
-                    if (m < g.M) Pz[static_cast<long>(m) * g.NN + n] = acc[tm][tn][e];
-                }
+                    for (int tn = 0; tn < 2; ++tn)
+                        acc[tm][tn] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[tm], bv[tn], acc[tm][tn], 0, 0, 0);
+            }
         }
     }
-    if (do_bias && tid < BM && m0 + tid < g.M)
-        g.Pb[static_cast<long>(z) * g.M + m0 + tid] = static_cast<float>(bsum);
+
+    // a lane's four consecutive rows of a column as one 16-byte store
+    const int mq = (g.M + 3) >> 2, npad = g.n_tiles * WG_BN;
+    float4* Pz = reinterpret_cast<float4*>(g.P) + static_cast<long>(z) * mq * npad;
+#pragma unroll
+    for (int tn = 0; tn < 2; ++tn) {
+        const int n = nt * WG_BN + (wn * 2 + tn) * 32 + l32;
+#pragma unroll
+        for (int tm = 0; tm < 2; ++tm)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int m4 = (m0 + wm * 64 + tm * 32 + 8 * j + 4 * hi) >> 2;
+                if (m4 < mq)
+                    Pz[static_cast<long>(m4) * npad + n] = make_float4(acc[tm][tn][4 * j], acc[tm][tn][4 * j + 1],
+                                                                       acc[tm][tn][4 * j + 2], acc[tm][tn][4 * j + 3]);
+            }
+    }
+    if (do_bias) {  // uniform: the four octets of a row sit in four neighbouring lanes
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            double t = bsum[i];
+            t += __shfl_xor(t, 1, 64);
+            t += __shfl_xor(t, 2, 64);
+            const int m = m0 + g_row + 64 * i;
+            if (g_oct == 0 && m < g.M) g.Pb[static_cast<long>(z) * g.M + m] = static_cast<float>(t);
+        }
+    }
 }
 
 // db[m] += sum_y part[y*M + m] (one wave per row, four rows per 256-thread
@@ -2146,70 +2183,63 @@ __device__ inline void bias_rows(const float* part, float* db, int M, int S, int
     if (lane == 0) db[m] += static_cast<float>(acc);
 }
 
-// out[i] += sum_z P[z][i] over the splits z, for V-float columns i (V = 4:
-// 16-byte accesses, MN a multiple of 4 and both arrays 16-B aligned; BLK:
-// the partials in the row-quad layout the GEMM stores 16 bytes at a time,
-// each column's four sums added to four rows of out). A
+// out[m][c*k + t] += sum_z P[z] over the splits z, a row quad of one column
+// per thread (16-byte loads), its four sums added to four rows of out. A
 // 256-thread block takes 256 / ZG columns and ZG split groups: thread (q, c)
 // sums its group's contiguous range of z in order, eight loads in flight
 // (each issued unconditionally from a clamped z, only its use bounded), and
 // the groups' sums are added in group order. The stage-1 weight grads have
 // hundreds of splits over a few thousand columns: the split groups turn one
-// long chain of memory round trips per column into ZG shorter ones. Blocks at
-// and past `main_blocks` (when Pb is given) sum the bias partials
+// long chain of memory round trips per column into ZG shorter ones. Columns
+// that stand for no (c, t) (a channel group's tail, taps past k) are skipped.
+// Blocks at and past `main_blocks` (when Pb is given) sum the bias partials
 // Pb[splits][M] into db instead, as bias_reduce would.
-template <int V, int ZG, bool BLK = false>
-__global__ __launch_bounds__(256) void wgrad_reduce(const float* P, float* out, long MN, int splits, int M,
-                                                    const float* Pb, float* db, unsigned main_blocks) {
+template <int ZG>
+__global__ __launch_bounds__(256) void wgrad_reduce(WgradArgs g, float* out, float* db, unsigned main_blocks) {
     if (blockIdx.x >= main_blocks) {
-        bias_rows(Pb, db, M, splits, static_cast<int>(blockIdx.x - main_blocks));
+        bias_rows(g.Pb, db, g.M, g.splits, static_cast<int>(blockIdx.x - main_blocks));
         return;
     }
-    using T = typename std::conditional<V == 4, float4, float>::type;
     constexpr int CW = 256 / ZG;
-    const T* Pv = reinterpret_cast<const T*>(P);
-    T* ov = reinterpret_cast<T*>(out);
-    const long MV = MN / V;
-    const int c = threadIdx.x % CW, q = threadIdx.x / CW;
-    const long i = static_cast<long>(blockIdx.x) * CW + c;
-    const long ic = i < MV ? i : MV - 1;
-    const int z0 = static_cast<int>(static_cast<long>(q) * splits / ZG);
-    const int z1 = static_cast<int>(static_cast<long>(q + 1) * splits / ZG);
-    T acc{};
+    const int npad = g.n_tiles * WG_BN;
+    const long MV = static_cast<long>((g.M + 3) >> 2) * npad;
+    const int cl = threadIdx.x % CW, q = threadIdx.x / CW;
+    const long i = static_cast<long>(blockIdx.x) * CW + cl;
+    const long mq = i / npad;
+    const int n = static_cast<int>(i - mq * npad);
+    const int nb = n >> 5, cg = nb / g.T;
+    const int v = cg * 32 + (n & 31), c = v / g.R;
+    const int t = (nb - cg * g.T) * g.R + (v - c * g.R);
+    const bool in = i < MV && nb < g.NB && c < g.C_x && t < g.k;
+    const float4* Pv = reinterpret_cast<const float4*>(g.P) + (in ? i : 0);
+    const int z0 = static_cast<int>(static_cast<long>(q) * g.splits / ZG);
+    const int z1 = in ? static_cast<int>(static_cast<long>(q + 1) * g.splits / ZG) : 0;
+    float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     for (int z = z0; z < z1; z += 8) {
-        T v[8];
+        float4 w[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = Pv[min(z + j, z1 - 1) * MV + ic];
+        for (int j = 0; j < 8; ++j) w[j] = Pv[min(z + j, z1 - 1) * MV];
 #pragma unroll
         for (int j = 0; j < 8; ++j)
-            if (z + j < z1) acc += v[j];
+            if (z + j < z1) acc += w[j];
     }
-    // BLK: P in row quads, column i = (m / 4) * NN + n holds rows m .. m + 3
-    auto put = [&](const T& t) {
-        if constexpr (BLK) {
-            const long NN = MN / M;
-            const long mq = i / NN, n = i - mq * NN;
-            float* o = out + 4 * mq * NN + n;
-            o[0] += t.x;
-            o[NN] += t.y;
-            o[2 * NN] += t.z;
-            o[3 * NN] += t.w;
-        } else {
-            ov[i] += t;
-        }
-    };
-    if constexpr (ZG == 1) {
-        if (i < MV) put(acc);
-    } else {
-        __shared__ T red[ZG][CW];
-        red[q][c] = acc;
+    if constexpr (ZG > 1) {
+        __shared__ float4 red[ZG][CW];
+        red[q][cl] = acc;
         __syncthreads();
-        if (q == 0 && i < MV) {
-            T t = red[0][c];
+        if (q == 0) {
 #pragma unroll
-            for (int g = 1; g < ZG; ++g) t += red[g][c];
-            put(t);
+            for (int u = 1; u < ZG; ++u) acc += red[u][cl];
         }
+    }
+    if (q == 0 && in) {
+        const long NN = static_cast<long>(g.C_x) * g.k;
+        const int m = static_cast<int>(mq) * 4;
+        float* o = out + m * NN + static_cast<long>(c) * g.k + t;
+        const float a[4] = {acc.x, acc.y, acc.z, acc.w};
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (m + u < g.M) o[u * NN] += a[u];
     }
 }
 
@@ -2927,68 +2957,22 @@ int kdec_conv1d_dgrad_adain_bwd(kdec_ctx* ctx, const float* W, const float* dY, 
                             dx_bs, dgamma, dbeta, dgb_bs, dalpha, N, C_in, L);
 }
 
-// LDS bytes of one wgrad_gemm block (two stages) and its input-row layout.
-struct WgradLayout {
-    int XR, span, segs, rs;
-    size_t lds;
-};
-
-WgradLayout wgrad_layout(int k, int s, int d, int wn) {
-    WgradLayout w{};
-    w.XR = (64 * wn - 1) / k + 2;
-    w.span = static_cast<int>(static_cast<long>(KC - 1) * s + static_cast<long>(k - 1) * d + 1);
-    w.segs = static_cast<int>(cdiv(w.span, 64));
-    // Column n = c*k + t sits at c*rs + t*d: with rs = k*d (mod 32) that is
-    // n*d (mod 32), distinct banks across 32 lanes for odd d; for k = 1 any
-    // odd rs. The smallest such rs >= span keeps the stage small (two blocks
-    // per CU for the k = 3 dilated convs).
-    long rs = w.span;
-    if (k == 1) {
-        if (rs % 2 == 0) ++rs;
-    } else {
-        const long want = (static_cast<long>(k) * d) % 32;
-        rs += ((want - rs % 32) % 32 + 32) % 32;
-    }
-    w.rs = static_cast<int>(rs);
-    // the packed staging writes whole 64-float runs: round the window up
-    const size_t xsz = (static_cast<size_t>(w.XR) * w.rs + 63) / 64 * 64;
-    w.lds = 2 * (static_cast<size_t>(64) * GP + xsz) * sizeof(float);
-    return w;
-}
-
-size_t wgrad_lds_bytes(int k, int s, int d, int wn) { return wgrad_layout(k, s, d, wn).lds; }
-
 #ifndef WG_ROUNDS
 #define WG_ROUNDS 2
 #endif
-const void* wgrad_kernel(bool s1, int wn) {
+const void* wgrad_kernel(bool s1) {
     static bool done = false;
-    const void* k[2][2] = {{reinterpret_cast<const void*>(&wgrad_gemm<false, 2>),
-                            reinterpret_cast<const void*>(&wgrad_gemm<false, 4>)},
-                           {reinterpret_cast<const void*>(&wgrad_gemm<true, 2>),
-                            reinterpret_cast<const void*>(&wgrad_gemm<true, 4>)}};
+    const void* k[2] = {reinterpret_cast<const void*>(&wgrad_gemm<false>),
+                        reinterpret_cast<const void*>(&wgrad_gemm<true>)};
     if (!done) {
-        for (auto& r : k)
-            for (const void* f : r)
-                (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        for (const void* f : k) (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         done = true;
     }
-    return k[s1 ? 1 : 0][wn == 4 ? 1 : 0];
+    return k[s1 ? 1 : 0];
 }
 
-// Waves along the column axis (C_x * k columns): the narrow 128-column tile
-// where it leaves fewer idle columns than the 256-column one (the stage-1
-// convs' 128 * {3, 7, 11} columns), else the wide tile.
-int wgrad_wn(int NN) {
-    const long w4 = cdiv(NN, 256) * 256 - NN, w2 = cdiv(NN, 128) * 128 - NN;
-    return w2 < w4 ? 2 : 4;
-}
-
-int wgrad_splits(kdec_ctx* ctx, int total_chunks, long tiles, size_t lds, bool s1, int wn) {
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, wgrad_kernel(s1, wn), 128 * wn, lds) != hipSuccess ||
-        per_cu < 1)
-        per_cu = 1;
+int wgrad_splits(kdec_ctx* ctx, int total_chunks, long tiles, size_t lds, bool s1) {
+    const int per_cu = blocks_per_cu(wgrad_kernel(s1), lds);
     // The most whole rounds of resident blocks, up to WG_ROUNDS, whose splits
     // keep at least 8 chunks each (shorter runs spend more on the partial
     // tile's write-out and reduction than on the GEMM); never a block past the
@@ -3003,79 +2987,60 @@ int wgrad_splits(kdec_ctx* ctx, int total_chunks, long tiles, size_t lds, bool s
 }
 
 // out (M x C_x*k) += the weight grad; db (M) += the row sums of G when
-// non-null (fused into the GEMM's n-tile-0 blocks).
+// non-null (fused into the GEMM's column-tile-0 blocks).
 static int wgrad_common(kdec_ctx* ctx, const float* X, long x_bs, const float* G,
                         long g_bs, int N, int M, int C_x, int L_x, int L_g, int k,
                         int s, int d, int p, float* out, float* db, const char* fam) {
-    const int NN = C_x * k;
-    const int wn = wgrad_wn(NN);
-    const int m_tiles = static_cast<int>(cdiv(M, BM));
-    const int n_tiles = static_cast<int>(cdiv(NN, 64 * wn));
-    const int chunks_per_n = static_cast<int>(cdiv(L_g, KC));
-    const int total_chunks = chunks_per_n * N;
-    // split the position chunks so that the blocks fill WG_ROUNDS rounds of
-    // the resident slots
-    const int splits = wgrad_splits(ctx, total_chunks, static_cast<long>(m_tiles) * n_tiles,
-                                    wgrad_lds_bytes(k, s, d, wn), s == 1, wn);
-    const long MN = static_cast<long>(M) * NN;
-    Workspace P(ctx, static_cast<size_t>(splits) * MN * sizeof(float));
-    Workspace Pb(ctx, db ? static_cast<size_t>(splits) * M * sizeof(float) : 0);
-    if (!P.p || (db && !Pb.p)) return KDEC_ENOMEM;
-    WgradArgs a{};
-    a.X = X; a.x_bs = x_bs; a.G = G; a.g_bs = g_bs; a.P = P.as<float>();
-    a.Pb = db ? Pb.as<float>() : nullptr;
-    a.M = M; a.C_x = C_x; a.L_x = L_x; a.L_g = L_g; a.k = k; a.s = s; a.d = d; a.p = p;
-    a.NN = NN; a.chunks_per_n = chunks_per_n; a.total_chunks = total_chunks;
-    a.splits = splits;
-    a.n_tiles = n_tiles;
-    a.m_tiles = m_tiles;
-    const WgradLayout lay = wgrad_layout(k, s, d, wn);
-    a.XR = lay.XR;
-    a.span = lay.span;
-    a.segs = lay.segs;
-    a.rs = lay.rs;
-    a.blk4 = M % 4 == 0 ? 1 : 0;
     if (static_cast<long>(L_x) * 4 > 0x7fffffffL || static_cast<long>(L_g) * 4 > 0x7fffffffL)
         return fail(ctx, KDEC_EINVAL, "wgrad: rows too long");
     if (static_cast<long>(M) * L_g * 4 > 0x7fffffffL || static_cast<long>(C_x) * L_x * 4 > 0x7fffffffL)
         return fail(ctx, KDEC_EINVAL, "wgrad: operand too large for one buffer descriptor");
-    const size_t lds = lay.lds;
-    if (lds > 160 * 1024) return fail(ctx, KDEC_EINVAL, "wgrad: tile does not fit LDS");
-    const long blocks = static_cast<long>(n_tiles) * m_tiles * splits;
+    WgradArgs a{};
+    a.X = X; a.x_bs = x_bs; a.G = G; a.g_bs = g_bs;
+    a.M = M; a.C_x = C_x; a.L_x = L_x; a.L_g = L_g; a.k = k; a.s = s; a.p = p;
+    const bool s1 = s == 1;
+    a.R = s1 ? 1 : d == 1 ? s : k;
+    a.rd = d;
+    a.T = static_cast<int>(cdiv(k, a.R));
+    a.sh = s1 ? d : 1;
+    const long NB = cdiv(static_cast<long>(C_x) * a.R, 32) * a.T;
+    const int m_tiles = static_cast<int>(cdiv(M, BM));
+    a.n_tiles = static_cast<int>(cdiv(NB, 4));
+    a.m_tiles = m_tiles;
+    a.NB = static_cast<int>(NB);
+    for (int nt = 0; nt < a.n_tiles; ++nt) a.rows = std::max(a.rows, wgrad_cols(nt, a.NB, a.T, a.sh).rows);
+    const size_t lds = 2 * 3 * (static_cast<size_t>(WG_GPL) + static_cast<size_t>(a.rows) * 64);
+    a.chunks_per_n = static_cast<int>(cdiv(L_g, KC));
+    a.total_chunks = a.chunks_per_n * N;
+    // split the position chunks so that the blocks fill WG_ROUNDS rounds of
+    // the resident slots
+    a.splits = wgrad_splits(ctx, a.total_chunks, static_cast<long>(m_tiles) * a.n_tiles, lds, s1);
+    const long MV = cdiv(M, 4) * a.n_tiles * WG_BN;
+    Workspace P(ctx, static_cast<size_t>(a.splits) * MV * 4 * sizeof(float));
+    Workspace Pb(ctx, db ? static_cast<size_t>(a.splits) * M * sizeof(float) : 0);
+    if (!P.p || (db && !Pb.p)) return KDEC_ENOMEM;
+    a.P = P.as<float>();
+    a.Pb = db ? Pb.as<float>() : nullptr;
+    const long blocks = static_cast<long>(a.n_tiles) * m_tiles * a.splits;
     {
+        const double NN = static_cast<double>(C_x) * k;
         ProfScope ps(ctx, fam, 2.0 * N * M * static_cast<double>(L_g) * NN,
-                     4.0 * (static_cast<double>(N) * C_x * L_x + static_cast<double>(N) * M * L_g +
-                            static_cast<double>(M) * NN));
+                     4.0 * (static_cast<double>(N) * C_x * L_x + static_cast<double>(N) * M * L_g + M * NN));
         void* args[] = {&a};
-        if (hipLaunchKernel(wgrad_kernel(s == 1, wn), dim3(static_cast<unsigned>(blocks)), dim3(128 * wn), args, lds,
-                            ctx->stream) != hipSuccess)
+        if (hipLaunchKernel(wgrad_kernel(s1), dim3(static_cast<unsigned>(blocks)), dim3(NT), args, lds, ctx->stream) !=
+            hipSuccess)
             return fail(ctx, KDEC_EHIP, std::string(fam) + ": launch failed");
         if (int rc2 = launch_check(ctx, fam)) return rc2;
     }
     // the weight-grad partials and, in extra blocks, the bias partials
     ProfScope ps(ctx, "wgrad_reduce", 0.0);
-    const bool blk = a.blk4 != 0;
-    const bool v4 = blk || (MN % 4 == 0 && ((reinterpret_cast<unsigned long long>(P.p) |
-                                             reinterpret_cast<unsigned long long>(out)) & 15) == 0);
-    const int zg = splits >= 64 ? 8 : splits >= 16 ? 4 : 1;
-    const long cols = v4 ? MN / 4 : MN;
-    const unsigned mb = static_cast<unsigned>(cdiv(cols, 256 / zg));
+    const int zg = a.splits >= 64 ? 8 : a.splits >= 16 ? 4 : 1;
+    unsigned mb = static_cast<unsigned>(cdiv(MV, 256 / zg));
     const unsigned bb = db ? static_cast<unsigned>(cdiv(M, 4)) : 0u;
-    const void* kern = blk ? (zg == 8   ? reinterpret_cast<const void*>(&wgrad_reduce<4, 8, true>)
-                              : zg == 4 ? reinterpret_cast<const void*>(&wgrad_reduce<4, 4, true>)
-                                        : reinterpret_cast<const void*>(&wgrad_reduce<4, 1, true>))
-                       : v4 ? (zg == 8   ? reinterpret_cast<const void*>(&wgrad_reduce<4, 8>)
-                             : zg == 4 ? reinterpret_cast<const void*>(&wgrad_reduce<4, 4>)
-                                       : reinterpret_cast<const void*>(&wgrad_reduce<4, 1>))
-                          : (zg == 8   ? reinterpret_cast<const void*>(&wgrad_reduce<1, 8>)
-                             : zg == 4 ? reinterpret_cast<const void*>(&wgrad_reduce<1, 4>)
-                                       : reinterpret_cast<const void*>(&wgrad_reduce<1, 1>));
-    const float* Pp = P.as<float>();
-    const float* Pbp = db ? Pb.as<float>() : nullptr;
-    long mn = MN;
-    int sp = splits, mrows = M;
-    unsigned mbk = mb;
-    void* args[] = {&Pp, &out, &mn, &sp, &mrows, &Pbp, &db, &mbk};
+    const void* kern = zg == 8   ? reinterpret_cast<const void*>(&wgrad_reduce<8>)
+                       : zg == 4 ? reinterpret_cast<const void*>(&wgrad_reduce<4>)
+                                 : reinterpret_cast<const void*>(&wgrad_reduce<1>);
+    void* args[] = {&a, &out, &db, &mb};
     if (hipLaunchKernel(kern, dim3(mb + bb), dim3(256), args, 0, ctx->stream) != hipSuccess)
         return fail(ctx, KDEC_EHIP, "wgrad_reduce: launch failed");
     return launch_check(ctx, "wgrad_reduce");

@@ -1,7 +1,8 @@
-"""The input grads on split bf16 terms (split_gemm), against float64 on the
-CPU, where their tiles and chunks end: channels about multiples of 16, output
-rows about 128, positions about 128, windows that take all taps in one chunk and
-those that don't, and operands a bf16 term cannot hold."""
+"""The input and weight grads on split bf16 terms (split_gemm, wgrad_gemm),
+against float64 on the CPU, where their tiles and chunks end: channels about
+multiples of 16 and 32, output rows about 128, positions about 128 and 32,
+windows that take all taps in one chunk and those that don't, and operands a
+bf16 term cannot hold."""
 import numpy as np
 import pytest
 import torch
@@ -71,5 +72,60 @@ def test_operands_past_bf16(K, value, where):
     got = y.double().cpu()
     assert torch.equal(got.isnan(), ref.isnan())
     assert torch.equal(got.isinf(), ref.isinf()) and torch.equal(got[ref.isinf()], ref[ref.isinf()])
+    f = ref.isfinite()
+    assert (got[f] - ref[f]).norm() <= TOL * ref[f].norm()
+
+
+@pytest.mark.parametrize("N,ci,co,L,k,s,d", [
+    (1, 1, 1, 1, 1, 1, 1), (2, 31, 3, 33, 3, 1, 1), (1, 33, 127, 32, 3, 1, 5), (3, 32, 130, 31, 7, 1, 3),
+    (1, 50, 128, 700, 11, 1, 5), (2, 20, 22, 257, 7, 1, 1), (1, 130, 64, 95, 1, 1, 1), (1, 9, 9, 900, 5, 1, 90),
+    (2, 22, 40, 601, 12, 6, 1), (1, 1, 1, 131, 3, 2, 1), (1, 18, 20, 300, 4, 3, 5), (1, 40, 12, 500, 2, 1, 33),
+    (1, 64, 128, 50001, 3, 1, 1),
+])
+def test_wgrad_edges(K, N, ci, co, L, k, s, d):
+    # column blocks of 32 channels by a tap (shared and separate windows), row
+    # quads past C_out, chunks of 32 positions that end inside one, the
+    # strided forms (a stride's phases as channels), and the bias sums
+    g = torch.Generator().manual_seed(ci * 1000 + L)
+    p = d * (k - 1) // 2
+    Lo = (L + 2 * p - d * (k - 1) - 1) // s + 1
+    x, dy = torch.randn(N, ci, L, generator=g), torch.randn(N, co, Lo, generator=g)
+    dw, db = torch.ones(co, ci, k, device="cuda"), torch.ones(co, device="cuda")
+    xg, dyg = x.cuda(), dy.cuda()
+    K.call("kdec_conv1d_wgrad", P(xg), ci * L, P(dyg), co * Lo, P(dw), P(db), N, ci, L, co, k, s, p, d)
+    xp = F.pad(x.double(), (p, p + s))
+    cols = torch.stack([xp[:, :, t * d:t * d + (Lo - 1) * s + 1:s] for t in range(k)], 2)
+    ref = 1.0 + torch.einsum("nml,nctl->mct", dy.double(), cols)
+    assert rel(dw, ref) <= TOL
+    assert rel(db, 1.0 + dy.double().sum((0, 2))) <= TOL
+
+
+@pytest.mark.parametrize("k,s,L", [(20, 10, 33), (12, 6, 130), (3, 4, 9)])
+def test_convt_wgrad_edges(K, k, s, L):
+    N, ci, co, p = 2, 130, 24, max(0, (k - s) // 2)
+    g = torch.Generator().manual_seed(k)
+    Lo = (L - 1) * s - 2 * p + k
+    x, dy = torch.randn(N, ci, L, generator=g), torch.randn(N, co, Lo, generator=g)
+    dw = torch.zeros(ci, co, k, device="cuda")
+    xg, dyg = x.cuda(), dy.cuda()
+    K.call("kdec_convt1d_wgrad", P(xg), ci * L, P(dyg), co * Lo, P(dw), None, N, ci, L, co, k, s, p, 0)
+    dp = F.pad(dy.double(), (p, p + s))
+    cols = torch.stack([dp[:, :, t:t + (L - 1) * s + 1:s] for t in range(k)], 2)
+    assert rel(dw, torch.einsum("nml,nctl->mct", x.double(), cols)) <= TOL
+
+
+@pytest.mark.parametrize("value,where", [(v, w) for v in (np.inf, np.nan, 3.4e38) for w in ("x", "dy")])
+def test_wgrad_operands_past_bf16(K, value, where):
+    N, ci, co, L, k, p = 1, 40, 130, 300, 3, 1
+    g = torch.Generator().manual_seed(6)
+    x, dy = torch.randn(N, ci, L, generator=g) * 0.1, torch.randn(N, co, L, generator=g) * 0.1
+    (x if where == "x" else dy)[0, 5, 150] = value
+    dw = torch.zeros(co, ci, k, device="cuda")
+    xg, dyg = x.cuda(), dy.cuda()
+    K.call("kdec_conv1d_wgrad", P(xg), ci * L, P(dyg), co * L, P(dw), None, N, ci, L, co, k, 1, p, 1)
+    xp = F.pad(x.double(), (p, p))
+    ref = torch.stack([sum(torch.matmul(dy[n].double(), xp[n, :, t:t + L].t()) for n in range(N)) for t in range(k)], 2)
+    got = dw.double().cpu()
+    assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got.isinf(), ref.isinf())
     f = ref.isfinite()
     assert (got[f] - ref[f]).norm() <= TOL * ref[f].norm()
