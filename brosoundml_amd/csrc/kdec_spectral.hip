@@ -714,6 +714,62 @@ __global__ void style_bwd_w_k(const float* style, long s_bs, const float* dout, 
     }
 }
 
+// dW and db as style_bwd_w_k (the same double sums in utterance order, so the
+// same bits), a block of 256 threads forming SWR * 1024 / S rows: lane j4 of a
+// row's S / 4 holds four columns of SWR rows, the styles and the block's
+// d(out) rows staged in LDS and read by each row's lanes together. Bound by
+// HBM (dW read and written, 38 MB for the decoder's 37 396 x 128): all of a
+// thread's dW loads are in flight while the sums are formed, 16 bytes each.
+// A thread per element spent its time on the index division and on 2 N
+// dependent loads: 34.8 us for 8 utterances,
+// 13 us here.
+constexpr int SWR = 4;
+__global__ __launch_bounds__(256) void style_bwd_w_rows_k(const float* style, long s_bs, const float* dout, long d_bs,
+                                                          float* dW, float* db, int N, int rows, int S) {
+    extern __shared__ float sw[];  // style [N][S], then d(out) [N][R]
+    const int S4 = S / 4, RP = 256 / S4, R = SWR * RP;
+    const int r0 = blockIdx.x * R;
+    const int j4 = threadIdx.x % S4, rr = threadIdx.x / S4;
+    float4 old[SWR];
+#pragma unroll
+    for (int u = 0; u < SWR; ++u) {
+        const int r = min(r0 + rr + u * RP, rows - 1);
+        old[u] = reinterpret_cast<const float4*>(dW + static_cast<long>(r) * S)[j4];
+    }
+    float* sg = sw + N * S;
+    for (int i = threadIdx.x; i < N * S; i += 256) sw[i] = style[(i / S) * s_bs + i % S];
+    for (int i = threadIdx.x; i < N * R; i += 256)
+        sg[i] = r0 + i % R < rows ? dout[(i / R) * d_bs + r0 + i % R] : 0.0f;
+    __syncthreads();
+    double acc[SWR][4], accb[SWR];
+#pragma unroll
+    for (int u = 0; u < SWR; ++u) acc[u][0] = acc[u][1] = acc[u][2] = acc[u][3] = accb[u] = 0.0;
+    for (int n = 0; n < N; ++n) {
+        const float4 t = reinterpret_cast<const float4*>(sw + n * S)[j4];
+#pragma unroll
+        for (int u = 0; u < SWR; ++u) {
+            const double g = sg[n * R + rr + u * RP];
+            acc[u][0] += g * t.x;
+            acc[u][1] += g * t.y;
+            acc[u][2] += g * t.z;
+            acc[u][3] += g * t.w;
+            accb[u] += g;
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < SWR; ++u) {
+        const int r = r0 + rr + u * RP;
+        if (r >= rows) continue;
+        float4 o = old[u];
+        o.x += static_cast<float>(acc[u][0]);
+        o.y += static_cast<float>(acc[u][1]);
+        o.z += static_cast<float>(acc[u][2]);
+        o.w += static_cast<float>(acc[u][3]);
+        reinterpret_cast<float4*>(dW + static_cast<long>(r) * S)[j4] = o;
+        if (db && j4 == 0) db[r] += static_cast<float>(accb[u]);
+    }
+}
+
 // The same projections reading each fc row once for all N utterances (the
 // wave-per-(row, utterance) kernels above read the fc block N times).
 //
@@ -1237,7 +1293,15 @@ int kdec_style_proj_bwd(kdec_ctx* ctx, const float* W, const float* style,
                            ctx->stream, part.as<float>(), nblk, dstyle, dstyle_bs, beta, N, S);
         if (int rc = launch_check(ctx, "style_bwd_x_reduce")) return rc;
     }
-    if (dW) {
+    // the row kernel where a row's quads divide a block, dW takes 16-byte
+    // accesses and the operands of all utterances fit 48 KB of LDS
+    const long wrows = S > 0 && S % 4 == 0 ? SWR * (1024L / S) : 0;
+    const long wlds = static_cast<long>(N) * (S + wrows) * static_cast<long>(sizeof(float));
+    if (dW && wrows > 0 && 1024 % S == 0 && wlds <= 48 * 1024 && (reinterpret_cast<unsigned long long>(dW) & 15) == 0) {
+        hipLaunchKernelGGL(style_bwd_w_rows_k, dim3(static_cast<unsigned>(cdiv(rows, wrows))), dim3(256),
+                           static_cast<size_t>(wlds), ctx->stream, style, style_bs, dout, dout_bs, dW, db, N, rows, S);
+        if (int rc = launch_check(ctx, "style_bwd_w_rows")) return rc;
+    } else if (dW) {
         hipLaunchKernelGGL(style_bwd_w_k, dim3(g1(static_cast<long>(rows) * S)), dim3(256), 0, ctx->stream,
                            style, style_bs, dout, dout_bs, dW, db, N, rows, S);
         if (int rc = launch_check(ctx, "style_bwd_w")) return rc;
