@@ -87,9 +87,12 @@ struct GemmArgs {
     int full_per_xcd, parts_per_xcd;  // block slots per XCD for each kind
     float* P;
     int ybuf;                // (C_out + BM) * L_y * 4 < 2^31: the epilogue addresses Y through a descriptor
-    // octet mode (corr_gemm): K chunk = one input-channel octet x up to G taps
-    int G, n_tg, n_oct, span8;  // taps per chunk, tap groups, octets, staged positions
-    int n_c16;               // split_gemm: 16-channel chunks (G taps at most each, n_tg tap groups); 0: another kernel
+    // corr_gemm: the split parts end at chunks of one octet x up to G taps;
+    // staged chunks of `no` octets x up to cg taps at an LDS row stride of
+    // spanp positions, nsub blocks per tile
+    // (serial: all parts of a tile in one block, tiles_per_xcd tiles per XCD)
+    int G, n_tg, n_oct, cg, no, spanp, nsub, serial, tiles_per_xcd;
+    int n_c16;               // split_gemm: 16-channel chunks (of up to G taps at most each, n_tg tap groups); 0: another kernel
     int quad;                // conv_gemm_q: weights packed in quads of k-steps (stride 1, k = KT)
     // Output placement (polyphase transposed convs): every column lands y_off
     // positions on (a left pad of the output rows, whose length L_y counts
@@ -210,8 +213,8 @@ __device__ inline void decode_tile(const GemmArgs& g, int tile, TileGeo& T) {
 // its L2) and then parts_per_xcd slots for split-tile parts; the whole-tile
 // rounds and the short split-part round are thus the same on every XCD.
 // Returns false for a padding slot.
-__device__ inline bool block_work(const GemmArgs& g, int& tile, int& part) {
-    const int x = blockIdx.x & 7, local = blockIdx.x >> 3;
+__device__ inline bool block_work_at(const GemmArgs& g, int local, int& tile, int& part) {
+    const int x = blockIdx.x & 7;
     if (local < g.full_per_xcd) {
         tile = x * g.full_per_xcd + local;
         part = -1;
@@ -224,23 +227,36 @@ __device__ inline bool block_work(const GemmArgs& g, int& tile, int& part) {
     return true;
 }
 
-// Tile epilogue shared by the GEMM kernels: lane owns column l32 and rows
+__device__ inline bool block_work(const GemmArgs& g, int& tile, int& part) {
+    return block_work_at(g, blockIdx.x >> 3, tile, part);
+}
+
+// As above with g.nsub consecutive blocks of an XCD on each tile.
+__device__ inline bool block_work_sub(const GemmArgs& g, int& tile, int& part, int& sub) {
+    const int local = blockIdx.x >> 3;
+    sub = local % g.nsub;
+    return block_work_at(g, local / g.nsub, tile, part);
+}
+
+// Tile epilogue shared by the GEMM kernels: the wave owns TM x TN MFMA tiles
+// from row mw and column nw of the block's tile on, a lane owns column l32 and rows
 // 8*(e/4) + 4*hi + e%4 of each 32x32 MFMA tile. A split part writes its raw
 // sums to its compact partial tile; a whole tile applies bias, residual,
 // scale and beta and stores Y.
-__device__ inline void store_tile(const GemmArgs& g, const TileGeo& T, int tile, int part, const f32x16 (&acc)[2][2],
-                                  int wm, int wn, int hi, int l32) {
+template <int TM, int TN>
+__device__ inline void store_tile(const GemmArgs& g, const TileGeo& T, int tile, int part, const f32x16 (&acc)[TM][TN],
+                                  int mw, int nw, int hi, int l32) {
     const int b = T.b, n_q = T.n_q, os = T.os, oo = T.oo, m0 = T.m0, q0 = T.q0;
     if (part >= 0) {  // raw sums of this chunk range, tile-local [m][q]
         float* Pt = g.P + (static_cast<long>(tile - g.full_tiles) * g.fsplit + part) * (BM * BN);
 #pragma unroll
-        for (int tn = 0; tn < 2; ++tn)
+        for (int tn = 0; tn < TN; ++tn)
 #pragma unroll
-            for (int tm = 0; tm < 2; ++tm)
+            for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) {
-                    const int ml = wm * 64 + tm * 32 + 8 * (e >> 2) + 4 * hi + (e & 3);
-                    Pt[ml * BN + wn * 64 + tn * 32 + l32] = acc[tm][tn][e];
+                    const int ml = mw + tm * 32 + 8 * (e >> 2) + 4 * hi + (e & 3);
+                    Pt[ml * BN + nw + tn * 32 + l32] = acc[tm][tn][e];
                 }
         return;
     }
@@ -260,7 +276,7 @@ __device__ inline void store_tile(const GemmArgs& g, const TileGeo& T, int tile,
         const __amdgpu_buffer_rsrc_t yr = uniform_rsrc(Yb, rowb);
         const __amdgpu_buffer_rsrc_t rr = uniform_rsrc(Rb ? Rb : Yb, Rb ? rowb : 0);
         const __amdgpu_buffer_rsrc_t br = uniform_rsrc(g.bias ? g.bias : Yb, g.bias ? g.C_out * 4 : 0);
-        const int mrow = m0 + wm * 64 + 4 * hi;  // the lane's first row
+        const int mrow = m0 + mw + 4 * hi;  // the lane's first row
         // Operand loads go in runs of eight elements under one uniform branch
         // each (bias, residual, old Y), so a run costs one memory round trip:
         // a load under a branch of its own is waited for at the branch's
@@ -268,12 +284,12 @@ __device__ inline void store_tile(const GemmArgs& g, const TileGeo& T, int tile,
         // registers and the accumulators fit without spilling.
         const bool hb = g.bias != nullptr, hr = Rb != nullptr, hy = g.beta != 0.0f;
 #pragma unroll
-        for (int tn = 0; tn < 2; ++tn) {
-            const int q = q0 + wn * 64 + tn * 32 + l32;
+        for (int tn = 0; tn < TN; ++tn) {
+            const int q = q0 + nw + tn * 32 + l32;
             if (q >= n_q) continue;
             const int vo = (mrow * Ly + q * os + oo) * 4;
 #pragma unroll
-            for (int tm = 0; tm < 2; ++tm) {
+            for (int tm = 0; tm < TM; ++tm) {
 #pragma unroll
                 for (int e0 = 0; e0 < 16; e0 += 8) {
                     float bv[8], rv[8], yv[8];
@@ -310,7 +326,7 @@ __device__ inline void store_tile(const GemmArgs& g, const TileGeo& T, int tile,
             }
             if (g.refl && q * os + oo == 1 + g.y_off) {  // the reflected column 0 (beta = 0)
 #pragma unroll
-                for (int tm = 0; tm < 2; ++tm) {
+                for (int tm = 0; tm < TM; ++tm) {
 #pragma unroll
                     for (int e = 0; e < 16; ++e) {
                         const int dm = tm * 32 + 8 * (e >> 2) + (e & 3);
@@ -328,15 +344,15 @@ __device__ inline void store_tile(const GemmArgs& g, const TileGeo& T, int tile,
         return;
     }
 #pragma unroll
-    for (int tn = 0; tn < 2; ++tn) {
-        const int q = q0 + wn * 64 + tn * 32 + l32;
+    for (int tn = 0; tn < TN; ++tn) {
+        const int q = q0 + nw + tn * 32 + l32;
         if (q >= n_q) continue;
         const long j = static_cast<long>(q) * os + oo;
 #pragma unroll
-        for (int tm = 0; tm < 2; ++tm) {
+        for (int tm = 0; tm < TM; ++tm) {
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
-                const int m = m0 + wm * 64 + tm * 32 + 8 * (e >> 2) + 4 * hi + (e & 3);
+                const int m = m0 + mw + tm * 32 + 8 * (e >> 2) + 4 * hi + (e & 3);
                 if (m >= g.C_out) continue;
                 float v = acc[tm][tn][e];
                 if (g.bias) v += g.bias[m];
@@ -773,7 +789,7 @@ void conv_gemm(GemmArgs g) {
         __syncthreads();
     }
 
-    store_tile(g, T, tile, part, acc, wm, wn, hi, l32);
+    store_tile(g, T, tile, part, acc, wm * 64, wn * 64, hi, l32);
 }
 
 // Stride-1 correlation of KT taps with the weights read 16 B per lane.
@@ -978,153 +994,259 @@ void conv_gemm_q(GemmArgs g) {
         if (part < 0)
             store_tile_stats(g, Te, acc, wm, wn, hi, l32);
         else
-            store_tile(g, Te, te, part, acc, wm, wn, hi, l32);
+            store_tile(g, Te, te, part, acc, wm * 64, wn * 64, hi, l32);
     } else {
-        store_tile(g, Te, te, part, acc, wm, wn, hi, l32);
+        store_tile(g, Te, te, part, acc, wm * 64, wn * 64, hi, l32);
     }
 }
 
-// Stride-1 correlation (conv forward, conv input-grad, each transposed-conv
-// phase) as an implicit GEMM whose operands are read 16 B per lane.
+// Stride-1 correlation (conv forward, each transposed-conv phase) as an
+// implicit GEMM on grids of less than one round of resident blocks.
 //
-// K runs over (input channel c, tap t). A chunk is one channel octet
-// o (c = 8o + 4h + e, h in {0, 1}, e in 0..3) times a group of up to G taps.
-// In one 32x32x2 MFMA step e of tap t, lanes of half h contribute
-// k = (8o + 4h + e, t), so each lane needs, per tap, four consecutive
-// channels: the weights are packed as [o][t][h][m_pad][4] (a chunk's rows
-// are whole 2 KB runs per (t, h) and a block's 128 columns), and the input
-// window is staged channels-last, [h][position][4], by a gathering DMA
-// (lane i of a 64-lane load fetches channel 4h + i%4 at position i/4 and
-// lands at LDS float i of the block). One ds_read_b128 then feeds four
-// MFMA steps: per tap a wave reads 2 A and 2 B vectors for 16 MFMAs.
-// Grid, tile order, split parts and epilogue as conv_gemm.
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4)))
+// K runs over steps s = (channel octet o, tap t), octet-major. A step is four
+// 32x32x2 MFMA steps: in step e, lanes of half h contribute k = (8o + 4h + e,
+// t), so a lane's operands of a step are four consecutive channels, read as 16
+// bytes: the weights packed as [o][t][h][m_pad][4] straight from L2 into
+// registers D steps ahead (every block of an m-tile reads the same panel), the
+// input window staged channels-last, [octet half][position][4], so that a tap
+// is a shift by whole 16-byte rows. A chunk of two octets (one where the
+// window of all taps is too long for three staging items per thread; then up
+// to cg taps) is loaded to registers while the one before it is multiplied: a
+// barrier per 2 k steps, against one per four taps of an octet, and none of
+// the input's four-byte gathers, when both operands went through LDS DMA.
+//
+// A block is four waves of 32 x 32 TN: 128 rows by 32 TN columns of a 128 x 128
+// tile, g.nsub blocks per tile. Serial (g.serial): the block runs all parts of
+// its tile, adding each part's sum to the total in part order, as tile_reduce
+// would: no partial tiles to write and read, no second kernel. Otherwise each
+// part is a block of its own. Either way, and for any tile width, the order of
+// every output's sum is the plan's: steps in order within parts delimited by
+// chunks of G taps.
+// Measured (whole call, packing and reduction with it), against blocks of a
+// whole tile with both operands DMA'd to LDS a quarter chunk at a time: 1090 ->
+// 1024 channels, k = 3, L = 21: 44 -> 28 us; 128 channels, k = 3 / 11, L =
+// 24121: 46 -> 30, 100 -> 78 us; 256 channels, k = 3, L = 3220: 38 -> 26 us.
+// Tile order and epilogue as conv_gemm.
+constexpr int CORR_ITEMS = 3;   // staging items (one octet half of one position) per thread
+template <int G, int TN>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(TN == 2 ? 3 : 4)))
 void corr_gemm(GemmArgs g) {
     extern __shared__ float smem[];
+    f32x4* lds = reinterpret_cast<f32x4*>(smem);
+    constexpr int COLS = 32 * TN;  // columns per block
+    constexpr int D = G > 0 ? G : 6 / TN;  // steps the weights run ahead
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave & 1, wn = wave >> 1;
     const int l32 = lane & 31, hi = lane >> 5;
+    const int mw = wave * 32;  // the wave's first row in the tile
 
-    int tile, part;
-    if (!block_work(g, tile, part)) return;  // uniform per block
+    int tile, part, sub;
+    if (g.serial) {  // an XCD's tiles are consecutive, as in block_work
+        const int local = blockIdx.x >> 3;
+        sub = local % g.nsub;
+        tile = (blockIdx.x & 7) * g.tiles_per_xcd + local / g.nsub;
+        part = -1;
+        if (tile >= g.full_tiles + g.split_tiles) return;  // uniform per block
+    } else if (!block_work_sub(g, tile, part, sub)) {
+        return;  // uniform per block
+    }
     TileGeo T;
     decode_tile(g, tile, T);
     const int k = T.k, d = T.d;
-    if (T.q0 >= T.n_q) return;  // uniform per block
+    const int c0 = sub * COLS;              // the block's first column in the tile
+    if (T.q0 + c0 >= T.n_q) return;         // uniform per block
 
-    const int G = g.G, n_tg = g.n_tg, span8 = g.span8;
-    const int a_st = G * 1024;             // A floats per stage: G taps x 2 halves x 128 x 4
-    const int stage = a_st + 8 * span8;    // + input window: 2 halves x span8 positions x 4
-    const float* Xb = g.X + static_cast<long>(T.b) * g.x_bs;
-    const __amdgpu_buffer_rsrc_t xrs = uniform_rsrc(Xb, g.C_in * g.L_in * 4);
-    const int x0 = T.q0 - T.p;             // input position of column q0 at tap 0
-    // weight staging: wave w copies quarter w of every (tap, half) run:
-    // half w>>1, 256-float piece w&1 of the block's 512 floats
-    const long a_row = 8L * g.m_pad;       // floats per (octet, tap) = 2 halves x m_pad x 4
-    const float* Aw = T.A + static_cast<long>(T.m0) * 4 + (wave >> 1) * g.m_pad * 4 + (wave & 1) * 256 + lane * 4;
-    const int a_lds = (wave >> 1) * 512 + (wave & 1) * 256;
-    // input staging: wave w fetches half w&1, 16-position blocks (w>>1) + 2j
-    const int nb = span8 >> 4;
-    const int lane_c = (wave & 1) * 4 + (lane & 3);
-    const int lane_p = lane >> 2;
-    const int x_lds = a_st + (wave & 1) * span8 * 4;
+    const int cg = G > 0 ? k : g.cg, no = G > 0 ? 2 : g.no;
+    const int span = COLS + (cg - 1) * d;   // staged positions
+    const int spanp = g.spanp;              // LDS row stride in positions (corr_stage)
+    const int bufsz = no * 2 * spanp;
+    const __amdgpu_buffer_rsrc_t xrs = uniform_rsrc(g.X + static_cast<long>(T.b) * g.x_bs, g.C_in * g.L_in * 4);
+    const int x0 = T.q0 + c0 - T.p;         // input position of the first column at tap 0
+    const int rowB = g.L_in * 4;
 
-    auto issue = [&](int o, int tg, int sb) {
-        const int t0 = tg * G;
-        const int gt = min(G, k - t0);
-        const float* Ag = Aw + (static_cast<long>(o) * k + t0) * a_row;
-        for (int j = 0; j < gt; ++j)
-            __builtin_amdgcn_global_load_lds(Ag + j * a_row, smem + sb + j * 1024 + a_lds, 16, 0, 0);
-        const int xs = x0 + t0 * d;
-        const int c = o * 8 + lane_c;
-        const bool inner = o * 8 + 8 <= g.C_in && xs >= 0 && xs + span8 <= g.L_in;  // uniform
-        for (int blk = wave >> 1; blk < nb; blk += 2) {
-            const int pos = xs + blk * 16 + lane_p;
-            const unsigned off = (inner || (c < g.C_in && pos >= 0 && pos < g.L_in))
-                                     ? static_cast<unsigned>(c * g.L_in + pos) * 4u : 0x80000000u;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, smem + sb + x_lds + blk * 64, 4,
-                                                     static_cast<int>(off), 0, 0, 0);
+    // items e = tid + 256 i: octet half e % (2 no), position e / (2 no)
+    const int hsh = no;
+    const int nitems = span << hsh;
+    f32x4 xr[CORR_ITEMS];
+    auto load_x = [&](int o, int t) {
+#pragma unroll
+        for (int i = 0; i < CORR_ITEMS; ++i) {
+            if (wave * 64 + i * NT >= nitems) continue;  // uniform
+            const int e = tid + i * NT, h = e & (2 * no - 1);
+            const int pos = x0 + t * d + (e >> hsh);
+            // past the row: an offset past the buffer reads 0; so do channels past C_in
+            unsigned off = pos >= 0 && pos < g.L_in ? static_cast<unsigned>((o * 8 + h * 4) * rowB + pos * 4) : 0x80000000u;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                xr[i][j] =
+                    __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrs, static_cast<int>(off), 0, 0));
+                off += rowB;
+            }
+        }
+    };
+    auto store_x = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < CORR_ITEMS; ++i) {
+            const int e = tid + i * NT;
+            if (e < nitems) lds[buf * bufsz + (e & (2 * no - 1)) * spanp + (e >> hsh)] = xr[i];
         }
     };
 
-    f32x16 acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+    // the parts this block runs, [p, pb) of nparts; their first and last step
+    const int nchunks = g.n_oct * g.n_tg;
+    const int nparts = tile < g.full_tiles ? 1 : g.fsplit;
+    int p = part < 0 ? 0 : part;
+    const int pb = part < 0 ? nparts : part + 1;
+    auto step_of = [&](int q) {
+        const int ch = q * nchunks / nparts;
+        return (ch / g.n_tg) * k + (ch % g.n_tg) * g.G;
+    };
+    int s = step_of(p), pe = step_of(p + 1);
+    const int s1 = step_of(pb);
 
-    const int nchunks = g.n_oct * n_tg;
-    const int nparts = part < 0 ? 1 : g.fsplit;
-    const int pp = part < 0 ? 0 : part;
-    const int ch0 = pp * nchunks / nparts;
-    const int ch1 = (pp + 1) * nchunks / nparts;
-    const bool live = T.q0 + wn * 64 < T.n_q;  // wave-uniform
-    // lane reads: A at m = wm*64 + tm*32 + l32, B at column n = wn*64 + tn*32 + l32 (+ tap shift)
-    const int a_rd = hi * 512 + (wm * 64 + l32) * 4;
-    const int b_rd = a_st + hi * span8 * 4 + (wn * 64 + l32) * 4;
-
-    int o = ch0 / n_tg, tg = ch0 - (ch0 / n_tg) * n_tg;  // chunk ch = o * n_tg + tg
-    if (ch0 < ch1) issue(o, tg, 0);
-    __builtin_amdgcn_s_waitcnt(0);  // staging loads landed in LDS
-    __syncthreads();
-    for (int ch = ch0; ch < ch1; ++ch) {
-        const int sb = ((ch - ch0) & 1) * stage;
-        const int no = tg + 1 == n_tg ? o + 1 : o, ntg = tg + 1 == n_tg ? 0 : tg + 1;
-        if (ch + 1 < ch1) issue(no, ntg, stage - sb);
-        const int gt = min(G, k - tg * G);
-        const int ab = sb + a_rd, bb = sb + b_rd;
-        auto ld = [&](int tl, float4 (&a)[2], float4 (&bv)[2]) {
-            tl = min(tl, gt - 1);
-            int ao = ab + tl * 1024, bo = bb + tl * d * 4;
-            // opaque offsets keep each tap's reads where they are placed
-            asm volatile("" : "+v"(ao), "+v"(bo));
-            a[0] = *reinterpret_cast<const float4*>(smem + ao);
-            a[1] = *reinterpret_cast<const float4*>(smem + ao + 128);
-            bv[0] = *reinterpret_cast<const float4*>(smem + bo);
-            bv[1] = *reinterpret_cast<const float4*>(smem + bo + 128);
-        };
-        auto mm = [&](const float4 (&a)[2], const float4 (&bv)[2]) {
-            const float a0[4] = {a[0].x, a[0].y, a[0].z, a[0].w};
-            const float a1[4] = {a[1].x, a[1].y, a[1].z, a[1].w};
-            const float b0[4] = {bv[0].x, bv[0].y, bv[0].z, bv[0].w};
-            const float b1[4] = {bv[1].x, bv[1].y, bv[1].z, bv[1].w};
+    f32x16 acc[1][TN], tot[1][TN];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[e], b0[e], acc[0][0], 0, 0, 0);
-                acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[e], b1[e], acc[0][1], 0, 0, 0);
-                acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[e], b0[e], acc[1][0], 0, 0, 0);
-                acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[e], b1[e], acc[1][1], 0, 0, 0);
-            }
-        };
-        float4 pa[2], pb[2], qa[2], qb[2];
-        ld(0, pa, pb);
-        int tl = live ? 0 : gt;  // a wave whose columns all lie past n_q only stages
-        for (; tl + 1 < gt; tl += 2) {
-            ld(tl + 1, qa, qb);
-            mm(pa, pb);
-            ld(tl + 2, pa, pb);
-            mm(qa, qb);
-            // (1 MFMA, 1 read) x 4, then 12 MFMAs; twice
-            for (int r = 0; r < 2; ++r) {
-                for (int i = 0; i < 4; ++i) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[0][j][e] = tot[0][j][e] = 0.0f;
+
+    if (s < s1) {
+        const float* Aw = T.A + (static_cast<long>(hi) * g.m_pad + T.m0 + mw + l32) * 4;
+        const long a_row = 8L * g.m_pad;
+        auto load_a = [&](int st) { return *reinterpret_cast<const f32x4*>(Aw + min(st, s1 - 1) * a_row); };
+        auto fold = [&]() {  // the part's sum onto the total
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    tot[0][j][e] += acc[0][j][e];
+                    acc[0][j][e] = 0.0f;
                 }
-                __builtin_amdgcn_sched_group_barrier(0x008, 12, 0);
+            ++p;
+            pe = step_of(min(p + 1, nparts));
+        };
+        auto load_b = [&](const f32x4* row, f32x4 (&b)[TN]) {
+#pragma unroll
+            for (int tn = 0; tn < TN; ++tn) b[tn] = row[tn * 32];
+        };
+        auto mma = [&](const f32x4& av, const f32x4 (&b)[TN]) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int tn = 0; tn < TN; ++tn)
+                    acc[0][tn] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[e], b[tn][e], acc[0][tn], 0, 0, 0);
+        };
+        if constexpr (G > 0) {
+            // chunks of two octets, all taps; the plan's chunks (up to G taps
+            // of an octet) unrolled, their weights one plan chunk ahead, the
+            // input a step ahead
+            int w = p * nchunks / nparts, we = (p + 1) * nchunks / nparts;
+            const int w1 = pb * nchunks / nparts;
+            int o = w / g.n_tg, tg = w - o * g.n_tg, co = o;
+            const int a_vo = (hi * g.m_pad + T.m0 + mw + l32) * 16, a_st = 32 * g.m_pad;
+            const int last = g.n_oct * k - 1;
+            f32x4 ring[D];
+            // weights of step st + u: the panel from st on through a descriptor, the step in the scalar offset
+            auto load_ring = [&](int st, int u, const __amdgpu_buffer_rsrc_t& ars) {
+                ring[u] = __builtin_bit_cast(
+                    f32x4, __builtin_amdgcn_raw_buffer_load_b128(ars, a_vo, min(u, last - st) * a_st, 0));
+            };
+            auto panel = [&](int st) { return uniform_rsrc(T.A + static_cast<long>(st) * (a_st / 4), 0x7fffffff); };
+            load_x(co, 0);
+            {
+                const __amdgpu_buffer_rsrc_t ars = panel(s);
+#pragma unroll
+                for (int u = 0; u < G; ++u) load_ring(s, u, ars);
+            }
+            store_x(0);
+            __syncthreads();
+            if ((w1 - 1) / g.n_tg >= co + 2) load_x(co + 2, 0);
+            int buf = 0;
+            for (; w < w1; ++w) {
+                const int gt = min(G, k - tg * G);
+                const int sn = min(s + gt, last);
+                const __amdgpu_buffer_rsrc_t ars = panel(sn);
+                const f32x4* row = lds + buf * bufsz + ((o - co) * 2 + hi) * spanp + l32 + tg * G * d;
+                f32x4 b[2][TN];
+                load_b(row, b[0]);
+#pragma unroll
+                for (int u = 0; u < G; ++u) {
+                    if (u + 1 < G) load_b(row + (u + 1 < gt ? u + 1 : 0) * d, b[(u + 1) & 1]);
+                    if (u == 0 || u < gt) mma(ring[u], b[u & 1]);  // uniform
+                    load_ring(sn, u, ars);
+                    __builtin_amdgcn_sched_barrier(0);  // nothing crosses into the next step
+                }
+                s += gt;
+                if (w + 1 == we) {
+                    fold();
+                    we = min(p + 1, nparts) * nchunks / nparts;
+                }
+                if (++tg == g.n_tg) {
+                    tg = 0;
+                    if (++o == co + 2 && w + 1 < w1) {
+                        co = o;
+                        buf ^= 1;
+                        store_x(buf);
+                        __syncthreads();
+                        if ((w1 - 1) / g.n_tg >= co + 2) load_x(co + 2, 0);
+                    }
+                }
+            }
+        } else {
+            // any k: as many octets and taps per chunk as the staging items hold
+            f32x4 ring[D];
+            // the chunk in hand: first octet, first tap, end step; the next one
+            int t = s % k;
+            int co = s / k, ct = cg == k ? 0 : t / cg * cg;
+            auto end_of = [&](int o, int tt) { return cg == k ? (o + no) * k : o * k + min(k, tt + cg); };
+            auto next = [&](int& o, int& tt) {
+                tt += cg;
+                if (tt >= k) {
+                    tt = 0;
+                    o += no;
+                }
+            };
+            int ce = end_of(co, ct);
+            load_x(co, ct);
+    #pragma unroll
+            for (int u = 0; u < D; ++u) ring[u] = load_a(s + u);
+            store_x(0);
+            __syncthreads();
+            int bo = hi * spanp + l32 + (t - ct) * d;
+            next(co, ct);
+            if (ce < s1) load_x(co, ct);
+            int buf = 0;
+            while (s < s1) {
+    #pragma unroll
+                for (int u = 0; u < D; ++u) {
+                    if (s >= s1) break;  // uniform
+                    f32x4 b[TN];
+                    load_b(lds + buf * bufsz + bo, b);
+                    mma(ring[u], b);
+                    ring[u] = load_a(s + D);
+                    ++s;
+                    bo += d;
+                    if (++t == k) {  // the next octet's half rows
+                        t = 0;
+                        bo += 2 * spanp - k * d;
+                    }
+                    if (s == pe) fold();
+                    if (s == ce && s < s1) {
+                        buf ^= 1;
+                        store_x(buf);
+                        __syncthreads();
+                        bo = hi * spanp + l32;
+                        ce = end_of(co, ct);
+                        next(co, ct);
+                        if (ce < s1) load_x(co, ct);
+                    }
+                }
             }
         }
-        if (live && tl < gt) mm(pa, pb);
-        o = no;
-        tg = ntg;
-        __builtin_amdgcn_s_waitcnt(0);  // this wave's staging loads landed
-        __syncthreads();
     }
 
-    store_tile(g, T, tile, part, acc, wm, wn, hi, l32);
+    store_tile(g, T, tile, part, tot, mw, c0, hi, l32);
 }
 
 // Stride-1 correlation on the bf16 matrix units at float precision: every
@@ -1314,7 +1436,7 @@ void split_gemm(GemmArgs g) {
         if (live) {
             const char* bp = lds + buf * stage + b_lane;
             const int nt = KT > 0 ? KT : min(G, k - (ch % n_tg) * G);
-#pragma unroll
+#pragma unroll KT > 0 ? KT : 1
             for (int t = 0; t < nt; ++t) {
                 bf16x8 an[3][2], b[3][2];
                 ++s;
@@ -1374,10 +1496,10 @@ void split_gemm(GemmArgs g) {
         if (part < 0) {  // uniform per block
             store_tile_adain(g, T, acc, wm, wn, hi, l32, smem);
         } else {
-            store_tile(g, T, tile, part, acc, wm, wn, hi, l32);
+            store_tile(g, T, tile, part, acc, wm * 64, wn * 64, hi, l32);
         }
     } else {
-        store_tile(g, T, tile, part, acc, wm, wn, hi, l32);
+        store_tile(g, T, tile, part, acc, wm * 64, wn * 64, hi, l32);
     }
 }
 
@@ -2546,23 +2668,49 @@ int blocks_per_cu(const void* kern, size_t lds) {
     return per_cu;
 }
 
+template <int G, int TN>
 const void* corr_kernel() {
     static bool attr = false;
     if (!attr) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&corr_gemm),
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&corr_gemm<G, TN>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         attr = true;
     }
-    return reinterpret_cast<const void*>(&corr_gemm);
+    return reinterpret_cast<const void*>(&corr_gemm<G, TN>);
 }
 
-// Octet-mode geometry for a stride-1 correlation of k taps at dilation d
-// over C channels: chunks of up to 4 taps (three for k = 3), the staged
-// window of a 4-tap chunk rounded to 16 positions.
-void octet_setup(GemmArgs& g, int C, int k, int d) {
+// The corr_gemm instance for k taps at dilation d and blocks of `cols`
+// columns, and its staging: two octets with the window of all taps where
+// CORR_ITEMS items per thread hold it (with k >= 3, the plan chunks unrolled),
+// else one octet with as many taps as they do.
+const void* corr_setup(GemmArgs& g, int cols, int k, int d) {
+    const long most = CORR_ITEMS * NT;
+    const bool all = 4 * (cols + static_cast<long>(k - 1) * d) <= most;
+    g.no = all ? 2 : 1;
+    g.cg = all ? k : static_cast<int>(std::min(static_cast<long>(k), (most / 2 - cols) / d + 1L));
+    // 4 / no mod 16: the staging stores of 2 no octet halves by 4 / no
+    // positions spread over the banks
+    const int sp = cols + (g.cg - 1) * d, want = 4 / g.no;
+    g.spanp = sp + ((want - sp % 16) + 16) % 16;
+    if (all && g.G == 3) return cols == 64 ? corr_kernel<3, 2>() : corr_kernel<3, 1>();
+    if (all && g.G == 4) return cols == 64 ? corr_kernel<4, 2>() : corr_kernel<4, 1>();
+    return cols == 64 ? corr_kernel<0, 2>() : corr_kernel<0, 1>();
+}
+
+// LDS bytes of a block that stages both operands of a plan chunk (G taps of an
+// octet) twice: what the split plan reckons its resident blocks with, and the
+// longest window that is taken. The parts' ends fix the order of the sums, so
+// the plan stays with this where the kernel stages less.
+long corr_plan_lds(int G, int d) {
+    const long span8 = cdiv(BN + static_cast<long>(G - 1) * d, 16) * 16;
+    return 2 * (G * 1024L + 8 * span8) * static_cast<long>(sizeof(float));
+}
+
+// Plan chunks of corr_gemm for a stride-1 correlation of k taps over C
+// channels: one octet x up to 4 taps (three for k = 3).
+void octet_setup(GemmArgs& g, int C, int k) {
     g.G = k < 4 ? k : 4;
     g.n_tg = static_cast<int>(cdiv(k, g.G));
-    g.span8 = static_cast<int>(cdiv(BN + (g.G - 1) * d, 16) * 16);
     g.n_oct = static_cast<int>(cdiv(C, 8));
     g.cin_pad = g.n_oct * 8;
     g.CK = 0;
@@ -2579,7 +2727,7 @@ void choose_chunks(kdec_ctx* ctx, GemmArgs& g, int C, int kk, int dd, long tiles
     const long slots = static_cast<long>(blocks_per_cu(conv_kernel_for(ck), conv_lds_bytes(ck, kk, 1, dd))) *
                        ctx->num_cus;
     if (tiles < slots) {
-        octet_setup(g, C, kk, dd);
+        octet_setup(g, C, kk);
         return;
     }
     g.G = 0;
@@ -2615,7 +2763,7 @@ int run_gemm(kdec_ctx* ctx, GemmArgs g, int N, int m_tiles, const char* fam,
     const int ss = g.n_phase > 1 ? 1 : g.s;
     const int dd = g.n_phase > 1 ? 1 : g.d;
     if (split ? (ss != 1 || g.G > kk || BN + static_cast<long>(g.G - 1) * dd > SPLIT_SPAN)
-        : octet ? (ss != 1 || g.G > kk || g.span8 < BN + (g.G - 1) * dd || g.span8 % 16)
+        : octet ? (ss != 1 || g.G > kk)
               : (CK * kk > 64 || (CK * kk) % 2))
         return fail(ctx, KDEC_EINVAL, "conv: bad chunk geometry");
     const bool quad = g.quad != 0;
@@ -2624,15 +2772,19 @@ int run_gemm(kdec_ctx* ctx, GemmArgs g, int N, int m_tiles, const char* fam,
         return fail(ctx, KDEC_EINVAL, "conv: no such epilogue in this kernel");
     if (quad && (octet || g.n_phase > 1 || g.s != 1 || !conv_q_kernel_for(CK, g.k, epi)))
         return fail(ctx, KDEC_EINVAL, "conv: bad quad geometry");
-    size_t lds = split ? split_lds_bytes(g.G, dd)
-               : octet ? 2 * (static_cast<size_t>(g.G) * 1024 + 8 * static_cast<size_t>(g.span8)) * sizeof(float)
-               : quad ? quad_lds_bytes(CK, g.k, g.d)
-                      : conv_lds_bytes(CK, kk, ss, dd);
+    // (corr_gemm's kernel and LDS follow from the plan)
+    size_t lds = split   ? split_lds_bytes(g.G, dd)
+                 : octet ? 0
+                 : quad  ? quad_lds_bytes(CK, g.k, g.d)
+                         : conv_lds_bytes(CK, kk, ss, dd);
     if (static_cast<long>(g.C_in) * g.L_in * 4 > 0x7fffffffL)
         return fail(ctx, KDEC_EINVAL, "conv: input too large for one buffer descriptor");
     g.ybuf = (static_cast<long>(g.C_out) + BM) * g.L_y * 4 < 0x7fffffffL ? 1 : 0;
-    const void* kern = split ? split_kernel_for(kk, g.G, epi) : octet ? corr_kernel() : quad ? conv_q_kernel_for(CK, g.k, epi) : conv_kernel_for(CK);
-    if (!kern) return fail(ctx, KDEC_EINVAL, "conv: unsupported channel chunk");
+    const void* kern = split   ? split_kernel_for(kk, g.G, epi)
+                       : octet ? nullptr
+                       : quad  ? conv_q_kernel_for(CK, g.k, epi)
+                               : conv_kernel_for(CK);
+    if (!kern && !octet) return fail(ctx, KDEC_EINVAL, "conv: unsupported channel chunk");
     // conv_gemm with one LDS stage where two leave at most two blocks per CU
     // and one leaves more (the long windows of large strides)
     g.single = 0;
@@ -2640,7 +2792,8 @@ int run_gemm(kdec_ctx* ctx, GemmArgs g, int N, int m_tiles, const char* fam,
         g.single = 1;
         lds /= 2;
     }
-    if (lds > 160 * 1024) return fail(ctx, KDEC_EINVAL, "conv: tile does not fit LDS");
+    if ((octet ? corr_plan_lds(g.G, dd) : static_cast<long>(lds)) > 160 * 1024)
+        return fail(ctx, KDEC_EINVAL, "conv: tile does not fit LDS");
     int max_q = g.n_q;
     if (g.n_phase > 1) max_q = static_cast<int>(cdiv(g.L_y + g.ph_s, g.ph_s)) + 1;
     g.m_tiles = m_tiles;
@@ -2648,7 +2801,9 @@ int run_gemm(kdec_ctx* ctx, GemmArgs g, int N, int m_tiles, const char* fam,
     g.nz = N * g.n_phase;
     const long tiles = static_cast<long>(g.m_tiles) * g.q_tiles * g.nz;
     if (tiles > 0x7fffffffL / 16) return fail(ctx, KDEC_EINVAL, "conv: grid too large");
-    const long slots = static_cast<long>(blocks_per_cu(kern, lds)) * ctx->num_cus;
+    // (three corr_gemm blocks per CU, or four where a plan chunk takes less than 40 KB)
+    const long per_cu = octet ? std::max(1L, std::min(4L, 160 * 1024 / corr_plan_lds(g.G, dd))) : blocks_per_cu(kern, lds);
+    const long slots = per_cu * ctx->num_cus;
     // a part keeps at least four chunks, of split_gemm at least eight steps (16 channels by one tap)
     const long parts = split ? std::min(static_cast<long>(g.n_c16) * g.n_tg, static_cast<long>(g.n_c16) * kk / 8)
                              : (octet ? g.n_oct * g.n_tg : g.cin_pad / CK) / 4;
@@ -2661,9 +2816,35 @@ int run_gemm(kdec_ctx* ctx, GemmArgs g, int N, int m_tiles, const char* fam,
     g.full_tiles = static_cast<int>(tiles - g.split_tiles);
     g.full_per_xcd = static_cast<int>(cdiv(g.full_tiles, 8));
     g.parts_per_xcd = static_cast<int>(cdiv(static_cast<long>(g.split_tiles) * g.fsplit, 8));
-    const long blocks = 8L * (g.full_per_xcd + g.parts_per_xcd);
-    Workspace part(ctx, static_cast<size_t>(g.split_tiles) * g.fsplit * BM * BN * sizeof(float));
-    if (g.split_tiles > 0) {
+    long blocks = 8L * (g.full_per_xcd + g.parts_per_xcd);
+    if (octet) {
+        // All parts in one block where the tiles alone keep the SIMDs busy for
+        // the length of their chain: a step of it takes 0.2 us with one wave
+        // per SIMD (twice its MFMAs), the parts' write-out and reduction
+        // 10-30 us. Measured, serial / parts: 128 -> 128 channels, k = 3, L =
+        // 24121 (189 tiles of 48 steps) 29.5 / 45.5 us, k = 11 (176 steps) 78
+        // / 91; 256 channels, k = 3, L = 3220 (52 of 96) 26 / 34, k = 11, L =
+        // 4000 (64 of 352) 72 / 72; 1024 -> 1024, k = 3, 8 x 100 (64 of 384)
+        // 98 / 88. Up to two taps (not unrolled, short chunks): 512 -> 256
+        // upsampler, 80 tiles of 128 steps 72 / 62, 400 tiles 167 / 175.
+        g.serial = f == 1 || static_cast<long>(g.n_oct) * kk * ctx->num_cus <= tiles * (g.G >= 3 ? 896 : 256);
+        // 64 columns per block where that leaves five blocks or more per four
+        // CUs (376 tiles of 352 steps: 270 us, with 32 columns 285; 126 tiles
+        // of 224 steps: 81, with 32 columns 77)
+        const long bt = g.serial ? tiles : tiles * f;
+        const int cols = max_q > 32 && bt * 4 >= 5L * ctx->num_cus ? 64 : 32;
+        kern = corr_setup(g, cols, kk, dd);
+        lds = 2 * 2 * static_cast<size_t>(g.no) * g.spanp * 16;
+        g.nsub = static_cast<int>(cdiv(std::min(max_q, BN), cols));
+        if (g.serial) {
+            g.tiles_per_xcd = static_cast<int>(cdiv(tiles, 8));
+            blocks = 8L * g.tiles_per_xcd;
+        }
+        blocks *= g.nsub;
+    }
+    const bool parted = g.split_tiles > 0 && !g.serial;  // partial tiles to reduce
+    Workspace part(ctx, parted ? static_cast<size_t>(g.split_tiles) * g.fsplit * BM * BN * sizeof(float) : 0);
+    if (parted) {
         if (!part.p) return KDEC_ENOMEM;
         g.P = part.as<float>();
     }
@@ -2686,7 +2867,7 @@ int run_gemm(kdec_ctx* ctx, GemmArgs g, int N, int m_tiles, const char* fam,
             return fail(ctx, KDEC_EHIP, std::string(fam) + ": launch failed");
         if (int rc = launch_check(ctx, fam)) return rc;
     }
-    if (g.split_tiles > 0) {
+    if (parted) {
         ProfScope ps(ctx, "tile_reduce", 0.0);
         if (g.ad.part)
             hipLaunchKernelGGL(tile_reduce_adain, dim3(BM * BN / 1024, g.split_tiles), dim3(256), 0, ctx->stream, g);
@@ -2850,6 +3031,17 @@ bool dgrad_fuses(kdec_ctx* ctx, int N, int C_in, int L) {
     return cdiv(C_in, BM) * cdiv(L, BN) * N >= 4L * ctx->num_cus;
 }
 
+// Whether a stride-1 window of k taps at dilation d is one that is taken (the
+// same as the forward's): the staged window of its kernel fits LDS.
+bool window_fits(kdec_ctx* ctx, int C, int k, int d, long tiles) {
+    GemmArgs g{};
+    choose_chunks(ctx, g, C, k, d, tiles);
+    const long lds = g.G > 0 ? corr_plan_lds(g.G, d)
+                     : pick_ck_q(k) > 0 ? static_cast<long>(quad_lds_bytes(pick_ck_q(k), k, d))
+                                        : static_cast<long>(conv_lds_bytes(g.CK, k, 1, d));
+    return lds <= 160 * 1024;
+}
+
 // The input grad as a correlation of dY with the flipped weights; with `ad`
 // (beta = 0) dX receives ds = dX * act'(s) of that AdaIN and
 // `part` its row partial sums (2 * q_tiles slots per row).
@@ -2874,6 +3066,7 @@ int conv_dgrad_impl(kdec_ctx* ctx, const float* W, const float* dY, long dy_bs, 
     g.k = k; g.s = 1; g.d = dil; g.p = pp; g.n_q = L;
     g.scale = scale; g.beta = beta; g.n_phase = 1;
     split_setup(g, C_out, k, dil);
+    KDEC_CHECK(ctx, window_fits(ctx, C_out, k, dil, cdiv(C_in, BM) * cdiv(L, BN) * N), "conv: tile does not fit LDS");
     if (ad) {
         if (beta != 0.0f) return fail(ctx, KDEC_EINVAL, "conv dgrad: no AdaIN epilogue for this geometry");
         g.ad.x = ad->X;
@@ -2995,6 +3188,14 @@ static int wgrad_common(kdec_ctx* ctx, const float* X, long x_bs, const float* G
         return fail(ctx, KDEC_EINVAL, "wgrad: rows too long");
     if (static_cast<long>(M) * L_g * 4 > 0x7fffffffL || static_cast<long>(C_x) * L_x * 4 > 0x7fffffffL)
         return fail(ctx, KDEC_EINVAL, "wgrad: operand too large for one buffer descriptor");
+    {  // the longest input window that is taken: the rows of 128 (256) columns, KC positions each, in half of LDS
+        const long NN = static_cast<long>(C_x) * k;
+        const long bn = cdiv(NN, 128) * 128 < cdiv(NN, 256) * 256 ? 128 : 256;
+        const long span = (KC - 1L) * s + (k - 1L) * d + 1;
+        const long rs = k == 1 ? span | 1 : span + ((static_cast<long>(k) * d - span) % 32 + 32) % 32;
+        if ((64 * 68 + cdiv(((bn - 1) / k + 2) * rs, 64) * 64) * 8 > 160 * 1024)
+            return fail(ctx, KDEC_EINVAL, "wgrad: tile does not fit LDS");
+    }
     WgradArgs a{};
     a.X = X; a.x_bs = x_bs; a.G = G; a.g_bs = g_bs;
     a.M = M; a.C_x = C_x; a.L_x = L_x; a.L_g = L_g; a.k = k; a.s = s; a.p = p;
