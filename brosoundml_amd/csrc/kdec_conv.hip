@@ -1289,18 +1289,17 @@ __device__ inline void split3(float x, __bf16& h, __bf16& m, __bf16& l) {
     l = static_cast<__bf16>(r - static_cast<float>(m));
 }
 
-__device__ inline void split_mma(const bf16x8 (&a)[3][2], const bf16x8 (&b)[3][2], f32x16 (&hh)[2][2],
-                                 f32x16 (&lo)[2][2]) {
-#define KDEC_SPLIT_MMA(ACC, I, J)                                                                       \
-    _Pragma("unroll") for (int tm = 0; tm < 2; ++tm) _Pragma("unroll") for (int tn = 0; tn < 2; ++tn)   \
-        ACC[tm][tn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[I][tm], b[J][tn], ACC[tm][tn], 0, 0, 0);
-    KDEC_SPLIT_MMA(lo, 0, 2)
-    KDEC_SPLIT_MMA(lo, 2, 0)
-    KDEC_SPLIT_MMA(lo, 1, 1)
-    KDEC_SPLIT_MMA(lo, 0, 1)
-    KDEC_SPLIT_MMA(lo, 1, 0)
-    KDEC_SPLIT_MMA(hh, 0, 0)
-#undef KDEC_SPLIT_MMA
+// One of a step's six products on the wave's 2 x 2 tiles, then a fence: the
+// loads written between two products stay there, the operand of a later step
+// under way while the products before it run.
+template <bool FENCE = true>
+__device__ inline void split_prod(const bf16x8 (&a)[2], const bf16x8 (&b)[2], f32x16 (&acc)[2][2]) {
+#pragma unroll
+    for (int tm = 0; tm < 2; ++tm)
+#pragma unroll
+        for (int tn = 0; tn < 2; ++tn)
+            acc[tm][tn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[tm], b[tn], acc[tm][tn], 0, 0, 0);
+    if (FENCE) __builtin_amdgcn_sched_barrier(0);
 }
 
 // The two accumulators' sum into hh; true where the wave has to form its sums
@@ -1402,13 +1401,14 @@ void split_gemm(GemmArgs g) {
     const int nsteps = g.n_c16 * k;
     const float* Ap = T.A + static_cast<long>(T.m0 / BM) * nsteps * SPLIT_STEP;
     const int a_lane = wm * 512 + lane * 4;  // floats
+    auto load_a1 = [&](int s, int pl, bf16x8 (&a)[2]) {
+        const float* p = Ap + static_cast<long>(s) * SPLIT_STEP + pl * 1024 + a_lane;
+#pragma unroll
+        for (int tm = 0; tm < 2; ++tm) a[tm] = *reinterpret_cast<const bf16x8*>(p + tm * 256);
+    };
     auto load_a = [&](int s, bf16x8 (&a)[3][2]) {
-        const float* p = Ap + static_cast<long>(s) * SPLIT_STEP;
 #pragma unroll
-        for (int pl = 0; pl < 3; ++pl)
-#pragma unroll
-            for (int tm = 0; tm < 2; ++tm)
-                a[pl][tm] = *reinterpret_cast<const bf16x8*>(p + pl * 1024 + tm * 256 + a_lane);
+        for (int pl = 0; pl < 3; ++pl) load_a1(s, pl, a[pl]);
     };
 
     f32x16 acc[2][2], lo[2][2];
@@ -1436,22 +1436,33 @@ void split_gemm(GemmArgs g) {
         if (live) {
             const char* bp = lds + buf * stage + b_lane;
             const int nt = KT > 0 ? KT : min(G, k - (ch % n_tg) * G);
+            bf16x8 b[3][2];
+            auto load_b = [&](int pl) {
+#pragma unroll
+                for (int tn = 0; tn < 2; ++tn)
+                    b[pl][tn] = *reinterpret_cast<const bf16x8*>(bp + pl * span * 32 + tn * 1024);
+            };
+#pragma unroll
+            for (int pl = 2; pl >= 0; --pl) load_b(pl);
 #pragma unroll KT > 0 ? KT : 1
             for (int t = 0; t < nt; ++t) {
-                bf16x8 an[3][2], b[3][2];
-                ++s;
-                load_a(min(s, s_end - 1), an);
-#pragma unroll
-                for (int pl = 2; pl >= 0; --pl)
-#pragma unroll
-                    for (int tn = 0; tn < 2; ++tn)
-                        b[pl][tn] = *reinterpret_cast<const bf16x8*>(bp + pl * span * 32 + tn * 1024);
-                split_mma(a, b, acc, lo);
-#pragma unroll
-                for (int pl = 0; pl < 3; ++pl)
-#pragma unroll
-                    for (int tm = 0; tm < 2; ++tm) a[pl][tm] = an[pl][tm];
-                bp += d * 32;
+                bf16x8 a0[2];  // the next step's first plane; the others reload in place
+                s = min(s + 1, s_end - 1);
+                if (t + 1 < nt) bp += d * 32;
+                load_a1(s, 0, a0);
+                split_prod(a[0], b[2], lo);
+                load_b(2);  // the next tap's, as each plane falls free
+                split_prod(a[2], b[0], lo);
+                load_a1(s, 2, a[2]);
+                split_prod(a[1], b[1], lo);
+                split_prod(a[1], b[0], lo);
+                load_a1(s, 1, a[1]);
+                split_prod(a[0], b[1], lo);
+                load_b(1);
+                split_prod(a[0], b[0], acc);
+                load_b(0);
+                a[0][0] = a0[0];
+                a[0][1] = a0[1];
             }
         }
         if (ch + 1 < ch1) store_x(buf ^ 1);
@@ -2204,26 +2215,58 @@ void wgrad_gemm(WgradArgs g) {
         if (ch + 1 < ch1) load(ch + 1);
         if (live) {
             const char* st = lds + buf * stage;
+            bf16x8 a[3][2], b[3][2];
+            auto load_a = [&](int ks, int pl, bf16x8 (&v)[2]) {
+#pragma unroll
+                for (int tm = 0; tm < 2; ++tm)
+                    v[tm] = *reinterpret_cast<const bf16x8*>(st + pl * WG_GPL + 2 * ks * WG_GO + a_rd + tm * 512);
+            };
+            auto load_b = [&](int ks, int pl) {
+#pragma unroll
+                for (int tn = 0; tn < 2; ++tn) {
+                    typedef short s16x4 __attribute__((ext_vector_type(4)));
+                    typedef __attribute__((address_space(3))) s16x4* LdsP;
+                    const char* p = st + pl * xpl + ks * 1024 + (tn ? b_rd1 : b_rd0);
+                    const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsP)(p));
+                    const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsP)(p + 256));
+                    b[pl][tn] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+                }
+            };
+            auto load_ab = [&](int ks) {
+                load_a(ks, 0, a[0]);
+                load_b(ks, 2);
+                load_a(ks, 2, a[2]);
+                load_b(ks, 0);
+                load_a(ks, 1, a[1]);
+                load_b(ks, 1);
+            };
+            load_ab(0);
 #pragma unroll
             for (int ks = 0; ks < KC / 16; ++ks) {
-                bf16x8 a[3][2], b[3][2];
-#pragma unroll
-                for (int pl = 0; pl < 3; ++pl)
-#pragma unroll
-                    for (int tm = 0; tm < 2; ++tm)
-                        a[pl][tm] = *reinterpret_cast<const bf16x8*>(st + pl * WG_GPL + 2 * ks * WG_GO + a_rd + tm * 512);
-#pragma unroll
-                for (int pl = 0; pl < 3; ++pl)
-#pragma unroll
-                    for (int tn = 0; tn < 2; ++tn) {
-                        typedef short s16x4 __attribute__((ext_vector_type(4)));
-                        typedef __attribute__((address_space(3))) s16x4* LdsP;
-                        const char* p = st + pl * xpl + ks * 1024 + (tn ? b_rd1 : b_rd0);
-                        const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsP)(p));
-                        const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsP)(p + 256));
-                        b[pl][tn] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
-                    }
-                split_mma(a, b, acc, lo);
+                // the next step's fragments as each plane falls free (the
+                // strided form has no registers left for that, nor for fences)
+                const bool more = S1 && ks + 1 < KC / 16;
+                bf16x8 a0[2];
+                split_prod<S1>(a[0], b[2], lo);
+                if (more) load_b(ks + 1, 2);
+                split_prod<S1>(a[2], b[0], lo);
+                if (more) load_a(ks + 1, 2, a[2]);
+                split_prod<S1>(a[1], b[1], lo);
+                split_prod<S1>(a[1], b[0], lo);
+                if (more) load_a(ks + 1, 1, a[1]);
+                split_prod<S1>(a[0], b[1], lo);
+                if (more) {
+                    load_b(ks + 1, 1);
+                    load_a(ks + 1, 0, a0);
+                }
+                split_prod<S1>(a[0], b[0], acc);
+                if (more) {
+                    load_b(ks + 1, 0);
+                    a[0][0] = a0[0];
+                    a[0][1] = a0[1];
+                } else if (ks + 1 < KC / 16) {
+                    load_ab(ks + 1);
+                }
             }
         }
         if (ch + 1 < ch1) store(buf ^ 1);
@@ -3151,7 +3194,7 @@ int kdec_conv1d_dgrad_adain_bwd(kdec_ctx* ctx, const float* W, const float* dY, 
 }
 
 #ifndef WG_ROUNDS
-#define WG_ROUNDS 2
+#define WG_ROUNDS 1
 #endif
 const void* wgrad_kernel(bool s1) {
     static bool done = false;
