@@ -1,8 +1,12 @@
 // Conv1d / ConvTranspose1d forward, input-grad and weight-grad on gfx950 as
 // implicit GEMMs on the matrix units, in float precision throughout: the
-// forwards and strided correlations on FP32 MFMA (v_mfma_f32_32x32x2_f32), the
-// stride-1 input grads on bf16 MFMA with every float split exactly into three
-// bf16 terms (split_gemm).
+// forwards on FP32 MFMA (v_mfma_f32_32x32x2_f32), the input and weight grads on
+// bf16 MFMA with every float split exactly into three bf16 terms (split_gemm,
+// wgrad_gemm: 1.4-1.9 times the rate, and closer to the exact sums). The
+// forwards stay on the float unit, and keep the order of every sum: the sign
+// of a pre-activation near a leaky kink decides its slope, so a forward that
+// rounds otherwise moves the gradients by up to 1e-3 (a few of 10^7 signs),
+// however small its own error.
 //
 // Forward family (one kernel, `conv_gemm`):
 //   Y[n, m, q] = sum_{c, t} A[(c, t), m] * X[n, c, q*s + t*d - p]
@@ -1274,7 +1278,12 @@ void corr_gemm(GemmArgs g) {
 // block of an XCD reads the same panel at about the same time.
 //
 // KT > 0: the tap count, all taps in one chunk. KT = 0: k at run time, chunks
-// of up to G taps so that any dilation's window fits.
+// of up to G taps so that any dilation's window fits. KT = -1: the input grad of
+// a transposed conv of stride s, k at run time: a stride's phases are channels,
+// v = (c, r) meeting position (q + t) s + r - p at tap t, so the strided
+// correlation of k taps is one of cdiv(k, s) taps at stride 1. The whole call at
+// 256 -> 512 channels, k = 20, s = 10, 4 x 5120, packing and reduction with it:
+// 138 us with the strided FP32 kernel, 90 here.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
@@ -1356,9 +1365,23 @@ void split_gemm(GemmArgs g) {
     const int rowB = g.L_in * 4;
     const bool two = wave * 64 + NT < 2 * span;  // wave-uniform: a second item
     float xr[2][8];
+    // Channel v's byte offset at the stride-1 position u; past the row an offset past the buffer.
+    auto strided_off = [&](int v, int u) {
+        const int c = v / g.s, ph = v - c * g.s;
+        const int pos = u * g.s + ph - g.p;
+        return pos >= 0 && pos < g.L_in ? static_cast<unsigned>(c * rowB + pos * 4) : 0x80000000u;
+    };
     auto load_item = [&](int i, int c16, int p0) {
         const int e = tid + i * NT;
         const int pos = p0 + (e >> 1);
+        if constexpr (KT < 0) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                xr[i][j] = __builtin_bit_cast(
+                    float, __builtin_amdgcn_raw_buffer_load_b32(
+                               xrs, static_cast<int>(strided_off(c16 * 16 + (e & 1) * 8 + j, pos)), 0, 0));
+            return;
+        }
         // past the row: an offset past the buffer reads 0; so do channels past C_in
         unsigned off = pos >= 0 && pos < g.L_in && e < 2 * span
                            ? static_cast<unsigned>((c16 * 16 + (e & 1) * 8) * rowB + pos * 4) : 0x80000000u;
@@ -1370,7 +1393,7 @@ void split_gemm(GemmArgs g) {
     };
     auto load_x = [&](int ch) {
         const int c16 = ch / n_tg, tg = ch - c16 * n_tg;
-        const int p0 = T.q0 - T.p + tg * G * d;
+        const int p0 = T.q0 - (KT < 0 ? 0 : T.p) + tg * G * d;
         load_item(0, c16, p0);
         if (two) load_item(1, c16, p0);
     };
@@ -1486,10 +1509,11 @@ void split_gemm(GemmArgs g) {
                     for (int u = 0; u < 2; ++u) {
                         av[u] = static_cast<float>(a[0][u][j]) +
                                 (static_cast<float>(a[1][u][j]) + static_cast<float>(a[2][u][j]));
-                        const int pos = T.q0 + wn * 64 + u * 32 + l32 - T.p + t * d;
-                        const unsigned off = pos >= 0 && pos < g.L_in
-                                                 ? static_cast<unsigned>((c16 * 16 + hi * 8 + j) * rowB + pos * 4)
-                                                 : 0x80000000u;
+                        const int q = T.q0 + wn * 64 + u * 32 + l32 + t * d, v = c16 * 16 + hi * 8 + j;
+                        const int pos = q - T.p;
+                        const unsigned off = KT < 0 ? strided_off(v, q)
+                                             : pos >= 0 && pos < g.L_in ? static_cast<unsigned>(v * rowB + pos * 4)
+                                                                        : 0x80000000u;
                         bv[u] = __builtin_bit_cast(
                             float, __builtin_amdgcn_raw_buffer_load_b32(xrs, static_cast<int>(off), 0, 0));
                     }
@@ -1824,22 +1848,6 @@ __global__ void pack_quad(const float* W, float* A, int C_in, int C_out, int k, 
     }
 }
 
-// conv-transpose input-grad: correlation over dY (C_out channels) with
-// A[(co, t), ci] = W[ci, co*k + t]
-__global__ void pack_convt_dgrad(const float* W, float* A, int C_in, int C_out,
-                                 int k, int cout_pad, int m_pad, int CK) {
-    const long total = static_cast<long>(cout_pad) * k * m_pad;
-    for (long i = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x; i < total;
-         i += static_cast<long>(gridDim.x) * blockDim.x) {
-        const int m = static_cast<int>(i % m_pad);  // ci
-        int c, t;                                   // c = co
-        panel_row(i / m_pad, CK, k, c, t);
-        float v = 0.0f;
-        if (m < C_in && c < C_out) v = W[(static_cast<long>(m) * C_out + c) * k + t];
-        A[i] = v;
-    }
-}
-
 // The panel row of (channel c, tap t) for CK-channel chunks, the inverse of
 // panel_row: row = ((c / CK) * kk + t) * CK + c % CK.
 __device__ inline long panel_index(int c, int t, int CK, int kk) {
@@ -1935,13 +1943,15 @@ __global__ void pack_octet(const float* W, float* A, int mode, int C_in, int C_o
 }
 
 // split_gemm's weight panel [m_tile][step = c16*k + t][plane][32-row block]
-// [lane][8] of a conv1d input-grad, A[(co, t), ci] = W[co, ci*k + k-1-t]: lane
+// [lane][8] of a conv1d input-grad (s = 0), A[(co, t), ci] = W[co, ci*k + k-1-t],
+// or of a transposed conv's at stride s, kt = cdiv(k, s) taps, channel (co, r):
+// A[(co, r, t), ci] = W[ci, co*k + t*s + r], zero where that is past k. Lane
 // (hi, l32) of block mb holds row ci = 32 mb + l32 of the tile, channels co =
 // 16 c16 + 8 hi + j, split in three bf16 planes; zero past either. One thread
 // per (step, block, lane). A weight that is not finite, or rounds past bf16's
 // range, keeps h + m + l = w (h truncated, or m = l = 0); one under 2^-110
 // keeps it to 2^-133, bf16's smallest step.
-__global__ void pack_split(const float* W, float* A, int C_in, int C_out, int k, int nsteps, long total) {
+__global__ void pack_split(const float* W, float* A, int C_in, int C_out, int k, int s, int kt, int nsteps, long total) {
     for (long i = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x; i < total;
          i += static_cast<long>(gridDim.x) * blockDim.x) {
         const unsigned iu = static_cast<unsigned>(i);  // total < 2^31 (the host's check of the panel size)
@@ -1949,14 +1959,19 @@ __global__ void pack_split(const float* W, float* A, int C_in, int C_out, int k,
         const unsigned rest = iu >> 8;
         const unsigned st = rest % static_cast<unsigned>(nsteps);
         const int mt = static_cast<int>(rest / static_cast<unsigned>(nsteps));
-        const int c16 = static_cast<int>(st) / k, t = static_cast<int>(st) - c16 * k;
+        const int c16 = static_cast<int>(st) / kt, t = static_cast<int>(st) - c16 * kt;
         const int m = mt * BM + mb * 32 + (lane & 31);
         const int c0 = c16 * 16 + (lane >> 5) * 8;
         float v[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const int c = c0 + j;
-            v[j] = m < C_in && c < C_out ? W[(static_cast<long>(c) * C_in + m) * k + (k - 1 - t)] : 0.0f;
+            if (s == 0) {
+                v[j] = m < C_in && c < C_out ? W[(static_cast<long>(c) * C_in + m) * k + (k - 1 - t)] : 0.0f;
+            } else {
+                const int co = c / s, tt = t * s + c - co * s;
+                v[j] = m < C_in && co < C_out && tt < k ? W[(static_cast<long>(m) * C_out + co) * k + tt] : 0.0f;
+            }
         }
         bf16x8 p[3];
 #pragma unroll
@@ -2646,9 +2661,10 @@ const void* split_kernel_epi(int epi) {
     return split_kernel<KT, QEPI_STORE>();
 }
 
-// The instance with the tap loop unrolled where all k taps' window fits one
+// The strided instance, or the one with the tap loop unrolled where all k taps' window fits one
 // chunk (the decoder's 3, 7 and 11), else the one that loops.
-const void* split_kernel_for(int k, int G, int epi) {
+const void* split_kernel_for(int k, int G, int epi, bool strided) {
+    if (strided) return split_kernel<-1, QEPI_STORE>();
     if (G == k && k == 3) return split_kernel_epi<3>(epi);
     if (G == k && k == 7) return split_kernel_epi<7>(epi);
     if (G == k && k == 11) return split_kernel_epi<11>(epi);
@@ -2805,12 +2821,12 @@ int run_gemm(kdec_ctx* ctx, GemmArgs g, int N, int m_tiles, const char* fam,
     const int kk = g.n_phase > 1 ? g.ph_kt : g.k;
     const int ss = g.n_phase > 1 ? 1 : g.s;
     const int dd = g.n_phase > 1 ? 1 : g.d;
-    if (split ? (ss != 1 || g.G > kk || BN + static_cast<long>(g.G - 1) * dd > SPLIT_SPAN)
+    const int epi = g.ad.part ? QEPI_ADAIN_BWD : g.fs.part ? QEPI_STATS : QEPI_STORE;
+    if (split ? ((ss != 1 && (dd != 1 || epi != QEPI_STORE)) || g.G > kk || BN + static_cast<long>(g.G - 1) * dd > SPLIT_SPAN)
         : octet ? (ss != 1 || g.G > kk)
               : (CK * kk > 64 || (CK * kk) % 2))
         return fail(ctx, KDEC_EINVAL, "conv: bad chunk geometry");
     const bool quad = g.quad != 0;
-    const int epi = g.ad.part ? QEPI_ADAIN_BWD : g.fs.part ? QEPI_STATS : QEPI_STORE;
     if (epi == QEPI_ADAIN_BWD ? !split : epi == QEPI_STATS && !quad)
         return fail(ctx, KDEC_EINVAL, "conv: no such epilogue in this kernel");
     if (quad && (octet || g.n_phase > 1 || g.s != 1 || !conv_q_kernel_for(CK, g.k, epi)))
@@ -2823,7 +2839,7 @@ int run_gemm(kdec_ctx* ctx, GemmArgs g, int N, int m_tiles, const char* fam,
     if (static_cast<long>(g.C_in) * g.L_in * 4 > 0x7fffffffL)
         return fail(ctx, KDEC_EINVAL, "conv: input too large for one buffer descriptor");
     g.ybuf = (static_cast<long>(g.C_out) + BM) * g.L_y * 4 < 0x7fffffffL ? 1 : 0;
-    const void* kern = split   ? split_kernel_for(kk, g.G, epi)
+    const void* kern = split   ? split_kernel_for(kk, g.G, epi, ss != 1)
                        : octet ? nullptr
                        : quad  ? conv_q_kernel_for(CK, g.k, epi)
                                : conv_kernel_for(CK);
@@ -3132,7 +3148,7 @@ int conv_dgrad_impl(kdec_ctx* ctx, const float* W, const float* dY, long dy_bs, 
                "kdec_conv1d_dgrad: weights too large");
     const long items = tot / SPLIT_STEP * 256;
     hipLaunchKernelGGL(pack_split, dim3(grid1d(items)), dim3(256), 0, ctx->stream, W, A.as<float>(), C_in, C_out, k,
-                       g.n_c16 * k, items);
+                       0, k, g.n_c16 * k, items);
     if (int rc = launch_check(ctx, "pack_dgrad")) return rc;
     return run_gemm(ctx, g, N, m_pad / BM, "conv_dgrad",
                     2.0 * N * C_out * static_cast<double>(L_out) * C_in * k);
@@ -3193,9 +3209,6 @@ int kdec_conv1d_dgrad_adain_bwd(kdec_ctx* ctx, const float* W, const float* dY, 
                             dx_bs, dgamma, dbeta, dgb_bs, dalpha, N, C_in, L);
 }
 
-#ifndef WG_ROUNDS
-#define WG_ROUNDS 1
-#endif
 const void* wgrad_kernel(bool s1) {
     static bool done = false;
     const void* k[2] = {reinterpret_cast<const void*>(&wgrad_gemm<false>),
@@ -3209,16 +3222,12 @@ const void* wgrad_kernel(bool s1) {
 
 int wgrad_splits(kdec_ctx* ctx, int total_chunks, long tiles, size_t lds, bool s1) {
     const int per_cu = blocks_per_cu(wgrad_kernel(s1), lds);
-    // The most whole rounds of resident blocks, up to WG_ROUNDS, whose splits
-    // keep at least 8 chunks each (shorter runs spend more on the partial
-    // tile's write-out and reduction than on the GEMM); never a block past the
-    // last whole round: blocks carry equal work (within one chunk), so one
-    // more would cost a whole extra round.
+    // One round of resident blocks, never a block past it (blocks carry equal
+    // work within one chunk, so one more would cost a whole extra round), and
+    // at least 8 chunks per split: shorter runs spend more on the partial
+    // tile's write-out and reduction than on the GEMM. Against two rounds: 84
+    // -> 75 us at 128 channels, k = 7, 2 x 24121; 978 -> 957 at k = 11, 8 x 61441.
     const long slots = static_cast<long>(ctx->num_cus) * per_cu;
-    for (int r = WG_ROUNDS; r >= 1; --r) {
-        const long splits = r * slots / tiles;
-        if (splits >= 1 && total_chunks / splits >= 8) return static_cast<int>(splits);
-    }
     return static_cast<int>(std::max(1L, std::min(slots / tiles, static_cast<long>(total_chunks / 8))));
 }
 
@@ -3256,8 +3265,7 @@ static int wgrad_common(kdec_ctx* ctx, const float* X, long x_bs, const float* G
     const size_t lds = 2 * 3 * (static_cast<size_t>(WG_GPL) + static_cast<size_t>(a.rows) * 64);
     a.chunks_per_n = static_cast<int>(cdiv(L_g, KC));
     a.total_chunks = a.chunks_per_n * N;
-    // split the position chunks so that the blocks fill WG_ROUNDS rounds of
-    // the resident slots
+    // split the position chunks so that the blocks fill one round
     a.splits = wgrad_splits(ctx, a.total_chunks, static_cast<long>(m_tiles) * a.n_tiles, lds, s1);
     const long MV = cdiv(M, 4) * a.n_tiles * WG_BN;
     Workspace P(ctx, static_cast<size_t>(a.splits) * MV * 4 * sizeof(float));
@@ -3420,26 +3428,28 @@ int kdec_convt1d_dgrad(kdec_ctx* ctx, const float* W, const float* dY,
                "kdec_convt1d_dgrad: bad arguments");
     const int L_out = (L - 1) * stride - 2 * pad + (k - 1) + op + 1;
     KDEC_CHECK(ctx, L > 0 && L_out > 0, "kdec_convt1d_dgrad: empty output");
+    // what the strided correlation kernel takes: the same windows as the forward's
     const int CK = pick_ck(k, stride, 1);
-    const int cpad = static_cast<int>(cdiv(C_out, 32) * 32);
-    const int m_pad = static_cast<int>(cdiv(C_in, BM) * BM);
-    const long tot = static_cast<long>(cpad) * k * m_pad;
+    KDEC_CHECK(ctx, CK * k <= 64, "conv: bad chunk geometry");
+    KDEC_CHECK(ctx, conv_lds_bytes(CK, k, stride, 1) <= 160 * 1024, "conv: tile does not fit LDS");
+    GemmArgs g{};
+    g.k = static_cast<int>(cdiv(k, stride));
+    KDEC_CHECK(ctx, static_cast<long>(C_out) * stride <= 0x7fffffffL - 16, "kdec_convt1d_dgrad: weights too large");
+    split_setup(g, C_out * stride, g.k, 1);
+    const long tot = split_panel(g, C_in);
+    KDEC_CHECK(ctx, tot <= 0x7fffffffL, "kdec_convt1d_dgrad: weights too large");
     Workspace A(ctx, static_cast<size_t>(tot) * sizeof(float));
     if (!A.p) return KDEC_ENOMEM;
-    if (cpad % CK == 0 && m_pad % 32 == 0)
-        hipLaunchKernelGGL(pack_rows_t, dim3(static_cast<unsigned>(cdiv(static_cast<long>(cpad) * k, 32)),
-                                             static_cast<unsigned>(m_pad / 32)),
-                           dim3(256), 0, ctx->stream, W, A.as<float>(), C_in, C_out, k, cpad, m_pad, CK);
-    else
-        hipLaunchKernelGGL(pack_convt_dgrad, dim3(grid1d(tot)), dim3(256), 0, ctx->stream, W, A.as<float>(),
-                           C_in, C_out, k, cpad, m_pad, CK);
+    const long items = tot / SPLIT_STEP * 256;
+    hipLaunchKernelGGL(pack_split, dim3(grid1d(items)), dim3(256), 0, ctx->stream, W, A.as<float>(), C_in, C_out, k,
+                       stride, g.k, g.n_c16 * g.k, items);
     if (int rc = launch_check(ctx, "pack_convt_dgrad")) return rc;
-    GemmArgs g{};
+    const int m_pad = static_cast<int>(cdiv(C_in, BM) * BM);
     g.X = dY; g.x_bs = dy_bs; g.A = A.as<float>();
     g.Y = dX; g.y_bs = dx_bs;
     g.C_in = C_out; g.L_in = L_out; g.C_out = C_in; g.L_y = L;
-    g.cin_pad = cpad; g.m_pad = m_pad;
-    g.k = k; g.s = stride; g.d = 1; g.p = pad; g.n_q = L; g.CK = CK;
+    g.m_pad = m_pad;
+    g.s = stride; g.d = 1; g.p = pad; g.n_q = L;
     g.scale = 1.0f; g.beta = 0.0f; g.n_phase = 1;
     return run_gemm(ctx, g, N, m_pad / BM, "convt_dgrad",
                     2.0 * N * C_in * static_cast<double>(L) * C_out * k);

@@ -129,3 +129,36 @@ def test_wgrad_operands_past_bf16(K, value, where):
     assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got.isinf(), ref.isinf())
     f = ref.isfinite()
     assert (got[f] - ref[f]).norm() <= TOL * ref[f].norm()
+
+
+@pytest.mark.parametrize("N,ci,co,k,s,L", [
+    (2, 130, 24, 20, 10, 33), (1, 127, 17, 12, 6, 130), (1, 9, 1, 3, 4, 9), (2, 20, 40, 5, 1, 140), (1, 64, 3, 7, 3, 257),
+])
+def test_convt_dgrad_edges(K, N, ci, co, k, s, L):
+    # a stride's phases as channels: k a multiple of the stride and not, taps
+    # past k, channels that end inside a chunk
+    g = torch.Generator().manual_seed(k)
+    p = max(0, (k - s) // 2)
+    Lo = (L - 1) * s - 2 * p + k
+    w, dy = torch.randn(ci, co * k, generator=g), torch.randn(N, co, Lo, generator=g)
+    dx = torch.full((N, ci, L), 7.0, device="cuda")
+    wg, dyg = w.cuda(), dy.cuda()
+    K.call("kdec_convt1d_dgrad", P(wg), P(dyg), co * Lo, P(dx), ci * L, N, ci, L, co, k, s, p, 0)
+    assert rel(dx, F.conv1d(dy.double(), w.double().reshape(ci, co, k), stride=s, padding=p)[..., :L]) <= TOL
+
+
+@pytest.mark.parametrize("value", [np.inf, np.nan, 3.4e38])
+def test_convt_dgrad_operands_past_bf16(K, value):
+    N, ci, co, k, s, p, L = 1, 40, 12, 12, 6, 3, 150
+    g = torch.Generator().manual_seed(7)
+    Lo = L * s
+    w, dy = torch.rand(ci, co * k, generator=g) * 0.2, torch.randn(N, co, Lo, generator=g)
+    dy[0, 3, 401] = value
+    dx = torch.empty(N, ci, L, device="cuda")
+    wg, dyg = w.cuda(), dy.cuda()
+    K.call("kdec_convt1d_dgrad", P(wg), P(dyg), co * Lo, P(dx), ci * L, N, ci, L, co, k, s, p, 0)
+    ref = F.conv1d(dy.double(), w.double().reshape(ci, co, k), stride=s, padding=p)
+    got = dx.double().cpu()
+    assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got.isinf(), ref.isinf())
+    f = ref.isfinite()
+    assert (got[f] - ref[f]).norm() <= TOL * ref[f].norm()
