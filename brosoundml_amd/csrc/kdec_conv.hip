@@ -2868,7 +2868,13 @@ int run_gemm(kdec_ctx* ctx, GemmArgs g, int N, int m_tiles, const char* fam,
                              : (octet ? g.n_oct * g.n_tg : g.cin_pad / CK) / 4;
     const long rem = tiles % slots;
     long f = 1;
-    if (rem > 0) f = std::min(std::min(slots / rem, parts), 16L);
+    // split_gemm tiles of few steps on many CUs stay whole: the parts' write-out
+    // and reduction cost more than the idle slots (128 channels, k = 3, 2 x 7681,
+    // 120 tiles of 24 steps: 34 us in parts, 26 whole; k = 7, 24121, 189 of 56:
+    // 53 / 43; k = 11, 2 x 7681, 120 of 88: 49 / 55; 256 channels, k = 7, 4000,
+    // 64 of 112: 40 / 46 in two)
+    const bool whole = split && 2L * g.n_c16 * kk * ctx->num_cus <= tiles * 256;
+    if (rem > 0 && !whole) f = std::min(std::min(slots / rem, parts), 16L);
     if (f < 2) f = 1;
     g.fsplit = static_cast<int>(f);
     g.split_tiles = f > 1 ? static_cast<int>(rem) : 0;
