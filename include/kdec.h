@@ -86,8 +86,8 @@ int kdec_conv1d_fwd(kdec_ctx* ctx, const float* X, long x_bs, const float* W,
 
 /* kdec_conv1d_fwd (beta = 0) that also writes the instance-norm statistics
  * of its output rows, stats[n*C_out + c] = (mean, 1/sqrt(var + eps)) as
- * kdec_instnorm_stats computes them. On grids of
- * four output tiles per CU or more the GEMM's epilogue records each tile's per-row count, mean and squared
+ * kdec_instnorm_stats computes them. Where the GEMM runs the quad-packed
+ * kernel, its epilogue records each tile's per-row count, mean and squared
  * deviations and a wave per row merges them (in double), so Y is not read
  * again; elsewhere it is the two calls. For the conv outputs that feed an
  * AdaIN (kokoro_decoder_backward.cpp:307-313, the ResBlock1 convs whose
@@ -115,8 +115,8 @@ int kdec_conv1d_dgrad(kdec_ctx* ctx, const float* W, const float* dY,
  * AdaIN + activation whose output feeds that conv:
  *   dX = kdec_adain_act_bwd(X, ..., dY' = conv1d_dgrad(W, dY)) (+ R)
  * with dgamma / dbeta overwritten and dalpha accumulated, as the two calls
- * kdec_conv1d_dgrad + kdec_adain_act_bwd (same arguments). On grids of
- * four output tiles per CU or more the GEMM's epilogue applies the activation
+ * kdec_conv1d_dgrad + kdec_adain_act_bwd (same arguments). On grids of four
+ * output tiles per CU or more, the GEMM's epilogue applies the activation
  * derivative and forms the AdaIN's per-row partial sums, so dY' is never
  * written separately and the AdaIN pass reads it once; elsewhere it makes
  * those two calls. dX must not alias X or R.
