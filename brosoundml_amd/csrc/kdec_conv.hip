@@ -97,6 +97,11 @@ struct GemmArgs {
     // (serial: all parts of a tile in one block, tiles_per_xcd tiles per XCD)
     int G, n_tg, n_oct, cg, no, spanp, nsub, serial, tiles_per_xcd;
     int n_c16;               // split_gemm: 16-channel chunks (of up to G taps at most each, n_tg tap groups); 0: another kernel
+    // split_gemm: the unpacked weights, for the sums it forms again on the
+    // float unit: a conv's [C_in][C_out][k], taps reversed (wk = 0), or a
+    // transposed conv's [C_out][C_in][wk]
+    const float* W;
+    int wk;
     int quad;                // conv_gemm_q: weights packed in quads of k-steps (stride 1, k = KT)
     // Output placement (polyphase transposed convs): every column lands y_off
     // positions on (a left pad of the output rows, whose length L_y counts
@@ -1257,8 +1262,8 @@ void corr_gemm(GemmArgs g) {
 // float operand is split exactly into three bf16 terms, x = h + m + l (8 + 8 +
 // 8 significant bits), and a product is the six bf16 products of order up to
 // 2^-16, accumulated in float: h h' in one accumulator, m h' + h m' + m m' +
-// l h' + h l' in a second that is added once at the end (the dropped terms lie
-// below 2^-26 of the product). The two accumulators keep the matrix unit's
+// l h' + h l' in a second that is added once at the end (the three products
+// dropped are at most 2^-24 of the product, 2^-27.5 rms). The two accumulators keep the matrix unit's
 // rounding of the small terms off the large sum: against double, over K = 16
 // .. 32768 random terms, 0.3-0.45 of v_mfma_f32_32x32x2's error, and none of
 // the downward bias that six products into one accumulator show (-8e-8 of the
@@ -1290,8 +1295,13 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 constexpr int SPLIT_STEP = 3 * BM * 16 / 2;  // floats of panel per (128 rows, step): three planes of 128 x 16 bf16
 constexpr int SPLIT_SPAN = 256;              // staged positions at most (two 8-channel items per thread)
 
-// x = h + m + l exactly (round to nearest each time, the last remainder fits).
+// 2^24 x = h + m + l exactly (round to nearest each time, the last remainder
+// fits), for every float under 2^104. The scale keeps the terms of the smallest
+// floats (multiples of 2^-149) normal: the matrix unit reads subnormal bf16 as
+// zero, so of a float of 2^-112 it would leave 16 bits, of 2^-124 four.
+constexpr float SPLIT_UP = 0x1p24f, SPLIT_DOWN = 0x1p-48f;
 __device__ inline void split3(float x, __bf16& h, __bf16& m, __bf16& l) {
+    x *= SPLIT_UP;
     h = static_cast<__bf16>(x);
     const float r = x - static_cast<float>(h);
     m = static_cast<__bf16>(r);
@@ -1311,12 +1321,11 @@ __device__ inline void split_prod(const bf16x8 (&a)[2], const bf16x8 (&b)[2], f3
     if (FENCE) __builtin_amdgcn_sched_barrier(0);
 }
 
-// The two accumulators' sum into hh; true where the wave has to form its sums
-// again on the float unit from the unsplit operands. An infinity splits as
-// inf + NaN + NaN, a float above the largest bf16 likewise, and the matrix
-// unit reads subnormal bf16 as zero, so the lower terms of operands under
-// 2^-110 are lost: a wave with a column that is not finite, or not zero yet
-// under 2^-90, goes back, and such inputs give what they give there.
+// The two accumulators' sum into hh, scaled back; true where the wave has to
+// form its sums again on the float unit from the unsplit operands: an operand
+// past 2^104 has infinite or NaN terms, and so has an infinity or a NaN
+// itself, and a sum past 2^80 overflows scaled. Such a wave goes back, and
+// these inputs give what they give there.
 __device__ inline bool split_finish(f32x16 (&hh)[2][2], const f32x16 (&lo)[2][2], bool live) {
     float mag = 0.0f;
 #pragma unroll
@@ -1325,10 +1334,10 @@ __device__ inline bool split_finish(f32x16 (&hh)[2][2], const f32x16 (&lo)[2][2]
         for (int j = 0; j < 2; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
-                hh[i][j][e] += lo[i][j][e];
+                hh[i][j][e] = (hh[i][j][e] + lo[i][j][e]) * SPLIT_DOWN;
                 mag += fabsf(hh[i][j][e]);
             }
-    return live && __any(!(mag <= 3.4028235e38f) || (mag > 0.0f && mag < 0x1p-90f));
+    return live && __any(!(mag <= 3.4028235e38f));
 }
 
 template <int KT, int EPI>
@@ -1498,18 +1507,21 @@ void split_gemm(GemmArgs g) {
             for (int j = 0; j < 2; ++j)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+        auto weight = [&](int m, int v, int t) {  // row m, channel v, tap t of the panel
+            if (g.wk == 0) return m < g.C_out && v < g.C_in ? g.W[(static_cast<long>(v) * g.C_out + m) * k + k - 1 - t] : 0.0f;
+            const int c = KT < 0 ? v / g.s : v, tt = KT < 0 ? t * g.s + v - c * g.s : t;
+            return m < g.C_out && c < g.C_in && tt < g.wk ? g.W[(static_cast<long>(m) * g.C_in + c) * g.wk + tt] : 0.0f;
+        };
         for (int ch = ch0; ch < ch1; ++ch) {
             const int c16 = ch / n_tg, tg = ch - c16 * n_tg;
             const int t1 = min(k, (tg + 1) * G);
             for (int t = tg * G; t < t1; ++t) {
-                load_a(c16 * k + t, a);
                 for (int j = 0; j < 8; ++j) {
                     float av[2], bv[2];
 #pragma unroll
                     for (int u = 0; u < 2; ++u) {
-                        av[u] = static_cast<float>(a[0][u][j]) +
-                                (static_cast<float>(a[1][u][j]) + static_cast<float>(a[2][u][j]));
                         const int q = T.q0 + wn * 64 + u * 32 + l32 + t * d, v = c16 * 16 + hi * 8 + j;
+                        av[u] = weight(T.m0 + wm * 64 + u * 32 + l32, v, t);
                         const int pos = q - T.p;
                         const unsigned off = KT < 0 ? strided_off(v, q)
                                              : pos >= 0 && pos < g.L_in ? static_cast<unsigned>(v * rowB + pos * 4)
@@ -1948,9 +1960,7 @@ __global__ void pack_octet(const float* W, float* A, int mode, int C_in, int C_o
 // A[(co, r, t), ci] = W[ci, co*k + t*s + r], zero where that is past k. Lane
 // (hi, l32) of block mb holds row ci = 32 mb + l32 of the tile, channels co =
 // 16 c16 + 8 hi + j, split in three bf16 planes; zero past either. One thread
-// per (step, block, lane). A weight that is not finite, or rounds past bf16's
-// range, keeps h + m + l = w (h truncated, or m = l = 0); one under 2^-110
-// keeps it to 2^-133, bf16's smallest step.
+// per (step, block, lane).
 __global__ void pack_split(const float* W, float* A, int C_in, int C_out, int k, int s, int kt, int nsteps, long total) {
     for (long i = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x; i < total;
          i += static_cast<long>(gridDim.x) * blockDim.x) {
@@ -1978,13 +1988,6 @@ __global__ void pack_split(const float* W, float* A, int C_in, int C_out, int k,
         for (int j = 0; j < 8; ++j) {
             __bf16 h, q, l;
             split3(v[j], h, q, l);
-            if (!(fabsf(static_cast<float>(h)) <= 3.4e38f)) {
-                const float tr = __uint_as_float(__float_as_uint(v[j]) & 0xffff0000u);
-                const bool fin = fabsf(v[j]) <= 3.4028235e38f;
-                h = static_cast<__bf16>(v[j] != v[j] ? v[j] : tr);
-                q = static_cast<__bf16>(fin ? v[j] - tr : 0.0f);
-                l = static_cast<__bf16>(fin ? (v[j] - tr) - static_cast<float>(q) : 0.0f);
-            }
             p[0][j] = h;
             p[1][j] = q;
             p[2][j] = l;
@@ -3130,6 +3133,7 @@ int conv_dgrad_impl(kdec_ctx* ctx, const float* W, const float* dY, long dy_bs, 
     g.m_pad = m_pad;
     g.k = k; g.s = 1; g.d = dil; g.p = pp; g.n_q = L;
     g.scale = scale; g.beta = beta; g.n_phase = 1;
+    g.W = W;
     split_setup(g, C_out, k, dil);
     KDEC_CHECK(ctx, window_fits(ctx, C_out, k, dil, cdiv(C_in, BM) * cdiv(L, BN) * N), "conv: tile does not fit LDS");
     if (ad) {
@@ -3457,6 +3461,8 @@ int kdec_convt1d_dgrad(kdec_ctx* ctx, const float* W, const float* dY,
     g.m_pad = m_pad;
     g.s = stride; g.d = 1; g.p = pad; g.n_q = L;
     g.scale = 1.0f; g.beta = 0.0f; g.n_phase = 1;
+    g.W = W;
+    g.wk = k;
     return run_gemm(ctx, g, N, m_pad / BM, "convt_dgrad",
                     2.0 * N * C_in * static_cast<double>(L) * C_out * k);
 }

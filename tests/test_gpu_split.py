@@ -25,7 +25,7 @@ def rel(a, r):
 
 # A float dot product of n terms of one sign pattern errs by at most n 2^-24 of
 # its terms' sum; the split one does no worse (24-bit operands, products to
-# 2^-26), so sqrt(n) 2^-24 of the result's norm bounds random terms: 2.2e-6 at
+# 2^-24 at worst and 2^-27.5 rms), so sqrt(n) 2^-24 of the result's norm bounds random terms: 2.2e-6 at
 # the most terms here (1408), stated for all.
 TOL = 2.5e-6
 
@@ -162,3 +162,58 @@ def test_convt_dgrad_operands_past_bf16(K, value):
     assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got.isinf(), ref.isinf())
     f = ref.isfinite()
     assert (got[f] - ref[f]).norm() <= TOL * ref[f].norm()
+
+
+def bounded(got, ref, mag, n):
+    # element by element: n terms of 24-bit operands err by at most n 2^-24 of
+    # the sum of their magnitudes, and a result under 2^-126 by float's last step
+    e = (got.double().cpu() - ref).abs()
+    return bool((e <= n * 2.0 ** -24 * mag + 2.0 ** -148).all())
+
+
+@pytest.mark.parametrize("e", [-104, -112, -118, -130])
+@pytest.mark.parametrize("where", ["positions", "row", "all"])
+@pytest.mark.parametrize("kind", ["dgrad", "convt_dgrad", "wgrad"])
+def test_tiny_operands(K, kind, where, e):
+    # operands about 2^e (subnormal ones too) in a few positions of the
+    # gradient, in one row of the weights (of the gradient for a weight grad,
+    # in one channel for "positions") or everywhere, beside ordinary ones: every
+    # result to float precision by itself
+    g = torch.Generator().manual_seed(-e)
+    t = 2.0 ** e
+    if kind == "wgrad":
+        N, ci, co, L, k = 2, 40, 130, 70, 3
+        x, dy = torch.randn(N, ci, L, generator=g), torch.randn(N, co, L, generator=g)
+        if where == "positions":
+            x[:, 5] *= t
+        elif where == "row":
+            dy[:, 70] *= t
+        else:
+            dy *= t
+            x *= 1e3
+        dw = torch.zeros(co, ci, k, device="cuda")
+        xg, dyg = x.cuda(), dy.cuda()
+        K.call("kdec_conv1d_wgrad", P(xg), ci * L, P(dyg), co * L, P(dw), None, N, ci, L, co, k, 1, 1, 1)
+        f = lambda x, dy: torch.stack([sum(dy[n] @ F.pad(x[n], (1, 1))[:, j:j + L].t() for n in range(N)) for j in range(k)], 2)
+        assert bounded(dw, f(x.double(), dy.double()), f(x.double().abs(), dy.double().abs()), N * L)
+        return
+    N, ci, co, L, k, s, p = (1, 130, 20, 300, 3, 1, 1) if kind == "dgrad" else (1, 130, 12, 150, 12, 6, 3)
+    Lo = L * s
+    dy = torch.randn(N, co, Lo, generator=g)
+    w = torch.randn(*((co, ci, k) if kind == "dgrad" else (ci, co, k)), generator=g)
+    if where == "positions":
+        dy[:, :, 140 * s:160 * s] *= t
+    elif where == "row":
+        (w[:, 70] if kind == "dgrad" else w[70]).mul_(t)
+    else:
+        dy *= t
+        w *= 1e3
+    dx = torch.empty(N, ci, L, device="cuda")
+    wg, dyg = w.cuda(), dy.cuda()
+    if kind == "dgrad":
+        K.call("kdec_conv1d_dgrad", P(wg), P(dyg), co * L, P(dx), ci * L, N, ci, L, co, k, 1, p, 1, 1.0, 0.0)
+        f = lambda w, dy: F.conv_transpose1d(dy, w, padding=p)
+    else:
+        K.call("kdec_convt1d_dgrad", P(wg), P(dyg), co * Lo, P(dx), ci * L, N, ci, L, co, k, s, p, 0)
+        f = lambda w, dy: F.conv1d(dy, w, stride=s, padding=p)
+    assert bounded(dx, f(w.double(), dy.double()), f(w.double().abs(), dy.double().abs()), co * k)
