@@ -3099,15 +3099,21 @@ bool dgrad_fuses(kdec_ctx* ctx, int N, int C_in, int L) {
     return cdiv(C_in, BM) * cdiv(L, BN) * N >= 4L * ctx->num_cus;
 }
 
-// Whether a stride-1 window of k taps at dilation d is one that is taken (the
-// same as the forward's): the staged window of its kernel fits LDS.
-bool window_fits(kdec_ctx* ctx, int C, int k, int d, long tiles) {
+// Whether an input grad of k taps at dilation d is taken: where the stride-1
+// forward of C channels and as many output tiles is. split_gemm itself runs any
+// window; the limits are the entry point's, kept from one kernel to the next:
+// grids of a round of conv_gemm's blocks or more take two channels' taps within
+// 64 weight rows (k <= 32), and every window fits the LDS of its forward kernel.
+int dgrad_taken(kdec_ctx* ctx, int C, int k, int d, long tiles) {
     GemmArgs g{};
     choose_chunks(ctx, g, C, k, d, tiles);
-    const long lds = g.G > 0 ? corr_plan_lds(g.G, d)
-                     : pick_ck_q(k) > 0 ? static_cast<long>(quad_lds_bytes(pick_ck_q(k), k, d))
-                                        : static_cast<long>(conv_lds_bytes(g.CK, k, 1, d));
-    return lds <= 160 * 1024;
+    const int ckq = g.G > 0 ? 0 : pick_ck_q(k);
+    if (g.G == 0 && g.CK * k > 64) return fail(ctx, KDEC_EINVAL, "conv: bad chunk geometry");
+    const long lds = g.G > 0   ? corr_plan_lds(g.G, d)
+                     : ckq > 0 ? static_cast<long>(quad_lds_bytes(ckq, k, d))
+                               : static_cast<long>(conv_lds_bytes(g.CK, k, 1, d));
+    if (lds > 160 * 1024) return fail(ctx, KDEC_EINVAL, "conv: tile does not fit LDS");
+    return KDEC_OK;
 }
 
 // The input grad as a correlation of dY with the flipped weights; with `ad`
@@ -3135,7 +3141,7 @@ int conv_dgrad_impl(kdec_ctx* ctx, const float* W, const float* dY, long dy_bs, 
     g.scale = scale; g.beta = beta; g.n_phase = 1;
     g.W = W;
     split_setup(g, C_out, k, dil);
-    KDEC_CHECK(ctx, window_fits(ctx, C_out, k, dil, cdiv(C_in, BM) * cdiv(L, BN) * N), "conv: tile does not fit LDS");
+    if (int rc = dgrad_taken(ctx, C_out, k, dil, cdiv(C_in, BM) * cdiv(L, BN) * N)) return rc;
     if (ad) {
         if (beta != 0.0f) return fail(ctx, KDEC_EINVAL, "conv dgrad: no AdaIN epilogue for this geometry");
         g.ad.x = ad->X;

@@ -217,3 +217,23 @@ def test_tiny_operands(K, kind, where, e):
         K.call("kdec_convt1d_dgrad", P(wg), P(dyg), co * Lo, P(dx), ci * L, N, ci, L, co, k, s, p, 0)
         f = lambda w, dy: F.conv1d(dy, w, stride=s, padding=p)
     assert bounded(dx, f(w.double(), dy.double()), f(w.double().abs(), dy.double().abs()), co * k)
+
+
+def test_dgrad_refusals(K):
+    # the forward's: more than 32 taps on a grid of a round of blocks or more,
+    # a window past LDS; on a small grid the taps are taken
+    def calls(N, c, L, k, d):
+        p = d * (k - 1) // 2
+        w, y = torch.ones(c, c * k, device="cuda"), torch.empty(N, c, L, device="cuda")
+        x = torch.ones_like(y)
+        yield lambda: K.call("kdec_conv1d_fwd", P(x), c * L, P(w), None, P(y), c * L, N, c, L, c, k, 1, p, d, None, 0, 1.0, 0.0)
+        yield lambda: K.call("kdec_conv1d_dgrad", P(w), P(x), c * L, P(y), c * L, N, c, L, c, k, 1, p, d, 1.0, 0.0)
+
+    for f in calls(1, 2, 128 * 4000, 33, 1):
+        with pytest.raises(native.KdecError, match="bad chunk geometry"):
+            f()
+    for f in calls(1, 2, 128 * 4000, 31, 800):
+        with pytest.raises(native.KdecError, match="does not fit LDS"):
+            f()
+    for f in calls(1, 2, 1000, 33, 1):
+        f()
