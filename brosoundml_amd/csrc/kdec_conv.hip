@@ -102,6 +102,7 @@ struct GemmArgs {
     // transposed conv's [C_out][C_in][wk]
     const float* W;
     int wk;
+    int nph;                 // phases of a channel (transposed convs of stride s > 1): min(s, wk)
     int quad;                // conv_gemm_q: weights packed in quads of k-steps (stride 1, k = KT)
     // Output placement (polyphase transposed convs): every column lands y_off
     // positions on (a left pad of the output rows, whose length L_y counts
@@ -1286,7 +1287,9 @@ void corr_gemm(GemmArgs g) {
 // of up to G taps so that any dilation's window fits. KT = -1: the input grad of
 // a transposed conv of stride s, k at run time: a stride's phases are channels,
 // v = (c, r) meeting position (q + t) s + r - p at tap t, so the strided
-// correlation of k taps is one of cdiv(k, s) taps at stride 1. The whole call at
+// correlation of k taps is one of cdiv(k, s) taps at stride 1. (r < min(s, k):
+// the other phases meet no tap. 512 -> 256, k = 1, s = 8, 4 x 2000: 195 us
+// with all eight, 38 with the one.) The whole call at
 // 256 -> 512 channels, k = 20, s = 10, 4 x 5120, packing and reduction with it:
 // 138 us with the strided FP32 kernel, 90 here.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -1376,7 +1379,7 @@ void split_gemm(GemmArgs g) {
     float xr[2][8];
     // Channel v's byte offset at the stride-1 position u; past the row an offset past the buffer.
     auto strided_off = [&](int v, int u) {
-        const int c = v / g.s, ph = v - c * g.s;
+        const int c = v / g.nph, ph = v - c * g.nph;
         const int pos = u * g.s + ph - g.p;
         return pos >= 0 && pos < g.L_in ? static_cast<unsigned>(c * rowB + pos * 4) : 0x80000000u;
     };
@@ -1509,7 +1512,7 @@ void split_gemm(GemmArgs g) {
                 for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
         auto weight = [&](int m, int v, int t) {  // row m, channel v, tap t of the panel
             if (g.wk == 0) return m < g.C_out && v < g.C_in ? g.W[(static_cast<long>(v) * g.C_out + m) * k + k - 1 - t] : 0.0f;
-            const int c = KT < 0 ? v / g.s : v, tt = KT < 0 ? t * g.s + v - c * g.s : t;
+            const int c = KT < 0 ? v / g.nph : v, tt = KT < 0 ? t * g.s + v - c * g.nph : t;
             return m < g.C_out && c < g.C_in && tt < g.wk ? g.W[(static_cast<long>(m) * g.C_in + c) * g.wk + tt] : 0.0f;
         };
         for (int ch = ch0; ch < ch1; ++ch) {
@@ -1956,12 +1959,13 @@ __global__ void pack_octet(const float* W, float* A, int mode, int C_in, int C_o
 
 // split_gemm's weight panel [m_tile][step = c16*k + t][plane][32-row block]
 // [lane][8] of a conv1d input-grad (s = 0), A[(co, t), ci] = W[co, ci*k + k-1-t],
-// or of a transposed conv's at stride s, kt = cdiv(k, s) taps, channel (co, r):
-// A[(co, r, t), ci] = W[ci, co*k + t*s + r], zero where that is past k. Lane
+// or of a transposed conv's at stride s, kt = cdiv(k, s) taps, channel (co, r <
+// R = min(s, k)): A[(co, r, t), ci] = W[ci, co*k + t*s + r], zero where that is past k. Lane
 // (hi, l32) of block mb holds row ci = 32 mb + l32 of the tile, channels co =
 // 16 c16 + 8 hi + j, split in three bf16 planes; zero past either. One thread
 // per (step, block, lane).
-__global__ void pack_split(const float* W, float* A, int C_in, int C_out, int k, int s, int kt, int nsteps, long total) {
+__global__ void pack_split(const float* W, float* A, int C_in, int C_out, int k, int s, int R, int kt,
+                           int nsteps, long total) {
     for (long i = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x; i < total;
          i += static_cast<long>(gridDim.x) * blockDim.x) {
         const unsigned iu = static_cast<unsigned>(i);  // total < 2^31 (the host's check of the panel size)
@@ -1979,7 +1983,7 @@ __global__ void pack_split(const float* W, float* A, int C_in, int C_out, int k,
             if (s == 0) {
                 v[j] = m < C_in && c < C_out ? W[(static_cast<long>(c) * C_in + m) * k + (k - 1 - t)] : 0.0f;
             } else {
-                const int co = c / s, tt = t * s + c - co * s;
+                const int co = c / R, tt = t * s + c - co * R;
                 v[j] = m < C_in && co < C_out && tt < k ? W[(static_cast<long>(m) * C_out + co) * k + tt] : 0.0f;
             }
         }
@@ -3164,7 +3168,7 @@ int conv_dgrad_impl(kdec_ctx* ctx, const float* W, const float* dY, long dy_bs, 
                "kdec_conv1d_dgrad: weights too large");
     const long items = tot / SPLIT_STEP * 256;
     hipLaunchKernelGGL(pack_split, dim3(grid1d(items)), dim3(256), 0, ctx->stream, W, A.as<float>(), C_in, C_out, k,
-                       0, k, g.n_c16 * k, items);
+                       0, 1, k, g.n_c16 * k, items);
     if (int rc = launch_check(ctx, "pack_dgrad")) return rc;
     return run_gemm(ctx, g, N, m_pad / BM, "conv_dgrad",
                     2.0 * N * C_out * static_cast<double>(L_out) * C_in * k);
@@ -3450,15 +3454,16 @@ int kdec_convt1d_dgrad(kdec_ctx* ctx, const float* W, const float* dY,
     KDEC_CHECK(ctx, conv_lds_bytes(CK, k, stride, 1) <= 160 * 1024, "conv: tile does not fit LDS");
     GemmArgs g{};
     g.k = static_cast<int>(cdiv(k, stride));
-    KDEC_CHECK(ctx, static_cast<long>(C_out) * stride <= 0x7fffffffL - 16, "kdec_convt1d_dgrad: weights too large");
-    split_setup(g, C_out * stride, g.k, 1);
+    g.nph = std::min(stride, k);
+    KDEC_CHECK(ctx, static_cast<long>(C_out) * g.nph <= 0x7fffffffL - 16, "kdec_convt1d_dgrad: weights too large");
+    split_setup(g, C_out * g.nph, g.k, 1);
     const long tot = split_panel(g, C_in);
     KDEC_CHECK(ctx, tot <= 0x7fffffffL, "kdec_convt1d_dgrad: weights too large");
     Workspace A(ctx, static_cast<size_t>(tot) * sizeof(float));
     if (!A.p) return KDEC_ENOMEM;
     const long items = tot / SPLIT_STEP * 256;
     hipLaunchKernelGGL(pack_split, dim3(grid1d(items)), dim3(256), 0, ctx->stream, W, A.as<float>(), C_in, C_out, k,
-                       stride, g.k, g.n_c16 * g.k, items);
+                       stride, g.nph, g.k, g.n_c16 * g.k, items);
     if (int rc = launch_check(ctx, "pack_convt_dgrad")) return rc;
     const int m_pad = static_cast<int>(cdiv(C_in, BM) * BM);
     g.X = dY; g.x_bs = dy_bs; g.A = A.as<float>();

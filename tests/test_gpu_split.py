@@ -133,10 +133,11 @@ def test_wgrad_operands_past_bf16(K, value, where):
 
 @pytest.mark.parametrize("N,ci,co,k,s,L", [
     (2, 130, 24, 20, 10, 33), (1, 127, 17, 12, 6, 130), (1, 9, 1, 3, 4, 9), (2, 20, 40, 5, 1, 140), (1, 64, 3, 7, 3, 257),
+    (1, 30, 33, 1, 8, 260), (2, 9, 5, 3, 10, 40), (1, 130, 16, 7, 8, 31),
 ])
 def test_convt_dgrad_edges(K, N, ci, co, k, s, L):
-    # a stride's phases as channels: k a multiple of the stride and not, taps
-    # past k, channels that end inside a chunk
+    # a stride's phases as channels: k a multiple of the stride and not, fewer
+    # taps than phases, taps past k, channels that end inside a chunk
     g = torch.Generator().manual_seed(k)
     p = max(0, (k - s) // 2)
     Lo = (L - 1) * s - 2 * p + k
