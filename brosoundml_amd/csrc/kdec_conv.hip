@@ -1968,7 +1968,7 @@ __global__ void pack_split(const float* W, float* A, int C_in, int C_out, int k,
                            int nsteps, long total) {
     for (long i = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x; i < total;
          i += static_cast<long>(gridDim.x) * blockDim.x) {
-        const unsigned iu = static_cast<unsigned>(i);  // total < 2^31 (the host's check of the panel size)
+        const unsigned iu = static_cast<unsigned>(i);  // total < 2^31: a 12th of the panel's floats (the host's checks)
         const int lane = iu & 63, mb = (iu >> 6) & 3;
         const unsigned rest = iu >> 8;
         const unsigned st = rest % static_cast<unsigned>(nsteps);
@@ -3103,12 +3103,14 @@ bool dgrad_fuses(kdec_ctx* ctx, int N, int C_in, int L) {
     return cdiv(C_in, BM) * cdiv(L, BN) * N >= 4L * ctx->num_cus;
 }
 
-// Whether an input grad of k taps at dilation d is taken: where the stride-1
-// forward of C channels and as many output tiles is. split_gemm itself runs any
-// window; the limits are the entry point's, kept from one kernel to the next:
-// grids of a round of conv_gemm's blocks or more take two channels' taps within
-// 64 weight rows (k <= 32), and every window fits the LDS of its forward kernel.
-int dgrad_taken(kdec_ctx* ctx, int C, int k, int d, long tiles) {
+// Whether an input grad to M channels of k taps at dilation d is taken: where
+// the stride-1 forward of C channels and as many output tiles is. split_gemm
+// itself runs any window, and panels of any size; the limits are the entry
+// point's, kept from one kernel to the next: grids of a round of conv_gemm's
+// blocks or more take two channels' taps within 64 weight rows (k <= 32), every
+// window fits the LDS of its forward kernel, and the float panel has under
+// 2^31 elements (split_gemm's takes half as many bytes again).
+int dgrad_taken(kdec_ctx* ctx, int C, int M, int k, int d, long tiles) {
     GemmArgs g{};
     choose_chunks(ctx, g, C, k, d, tiles);
     const int ckq = g.G > 0 ? 0 : pick_ck_q(k);
@@ -3117,6 +3119,11 @@ int dgrad_taken(kdec_ctx* ctx, int C, int k, int d, long tiles) {
                      : ckq > 0 ? static_cast<long>(quad_lds_bytes(ckq, k, d))
                                : static_cast<long>(conv_lds_bytes(g.CK, k, 1, d));
     if (lds > 160 * 1024) return fail(ctx, KDEC_EINVAL, "conv: tile does not fit LDS");
+    const long m_tiles = cdiv(M, BM);
+    const long tot = ckq > 0 ? m_tiles * (g.cin_pad / ckq) * cdiv(static_cast<long>(ckq) * k / 2, 4) * 1024
+                             : m_tiles * BM * static_cast<long>(g.cin_pad) * k;
+    KDEC_CHECK(ctx, tot <= 0x7fffffffL && static_cast<long>(M) * C * k <= 0x7fffffffL,
+               "kdec_conv1d_dgrad: weights too large");
     return KDEC_OK;
 }
 
@@ -3145,7 +3152,7 @@ int conv_dgrad_impl(kdec_ctx* ctx, const float* W, const float* dY, long dy_bs, 
     g.scale = scale; g.beta = beta; g.n_phase = 1;
     g.W = W;
     split_setup(g, C_out, k, dil);
-    if (int rc = dgrad_taken(ctx, C_out, k, dil, cdiv(C_in, BM) * cdiv(L, BN) * N)) return rc;
+    if (int rc = dgrad_taken(ctx, C_out, C_in, k, dil, cdiv(C_in, BM) * cdiv(L, BN) * N)) return rc;
     if (ad) {
         if (beta != 0.0f) return fail(ctx, KDEC_EINVAL, "conv dgrad: no AdaIN epilogue for this geometry");
         g.ad.x = ad->X;
@@ -3164,8 +3171,6 @@ int conv_dgrad_impl(kdec_ctx* ctx, const float* W, const float* dY, long dy_bs, 
     Workspace A(ctx, static_cast<size_t>(tot) * sizeof(float));
     if (!A.p) return KDEC_ENOMEM;
     g.A = A.as<float>();
-    KDEC_CHECK(ctx, tot <= 0x7fffffffL && static_cast<long>(C_out) * C_in * k <= 0x7fffffffL,
-               "kdec_conv1d_dgrad: weights too large");
     const long items = tot / SPLIT_STEP * 256;
     hipLaunchKernelGGL(pack_split, dim3(grid1d(items)), dim3(256), 0, ctx->stream, W, A.as<float>(), C_in, C_out, k,
                        0, 1, k, g.n_c16 * k, items);
@@ -3458,7 +3463,7 @@ int kdec_convt1d_dgrad(kdec_ctx* ctx, const float* W, const float* dY,
     KDEC_CHECK(ctx, static_cast<long>(C_out) * g.nph <= 0x7fffffffL - 16, "kdec_convt1d_dgrad: weights too large");
     split_setup(g, C_out * g.nph, g.k, 1);
     const long tot = split_panel(g, C_in);
-    KDEC_CHECK(ctx, tot <= 0x7fffffffL, "kdec_convt1d_dgrad: weights too large");
+    KDEC_CHECK(ctx, tot / 12 <= 0x7fffffffL, "kdec_convt1d_dgrad: weights too large");  // pack_split's items
     Workspace A(ctx, static_cast<size_t>(tot) * sizeof(float));
     if (!A.p) return KDEC_ENOMEM;
     const long items = tot / SPLIT_STEP * 256;

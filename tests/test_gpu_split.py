@@ -238,3 +238,21 @@ def test_dgrad_refusals(K):
             f()
     for f in calls(1, 2, 1000, 33, 1):
         f()
+
+
+@pytest.mark.parametrize("kind", ["dgrad", "convt_dgrad"])
+def test_large_weights(K, kind):
+    # 1.6e9 weights: within 2^31 as floats, past it as split panels
+    ci, co, k, s = (32768, 50000, 1, 1) if kind == "dgrad" else (32768, 25000, 2, 2)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    w = torch.randn(*((co, ci) if kind == "dgrad" else (ci, co * k)), generator=g, device="cuda")
+    dy = torch.randn(1, co, k, generator=g, device="cuda")
+    dx = torch.empty(1, ci, 1, device="cuda")
+    if kind == "dgrad":
+        K.call("kdec_conv1d_dgrad", P(w), P(dy), co, P(dx), ci, 1, ci, 1, co, 1, 1, 0, 1, 1.0, 0.0)
+        ref = sum(w[c:c + 2000].double().t() @ dy[0, c:c + 2000, 0].double() for c in range(0, co, 2000))
+    else:
+        K.call("kdec_convt1d_dgrad", P(w), P(dy), co * k, P(dx), ci, 1, ci, 1, co, k, s, 0, 0)
+        ref = torch.cat([w[m:m + 2048].double() @ dy.double().reshape(-1) for m in range(0, ci, 2048)])
+    # 50 000 terms: sqrt(n) 2^-24
+    assert rel(dx.reshape(-1), ref.cpu()) <= 1.4e-5
