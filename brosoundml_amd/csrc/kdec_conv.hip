@@ -1381,7 +1381,7 @@ void split_gemm(GemmArgs g) {
     auto strided_off = [&](int v, int u) {
         const int c = v / g.nph, ph = v - c * g.nph;
         const int pos = u * g.s + ph - g.p;
-        return pos >= 0 && pos < g.L_in ? static_cast<unsigned>(c * rowB + pos * 4) : 0x80000000u;
+        return c < g.C_in && pos >= 0 && pos < g.L_in ? static_cast<unsigned>(c * rowB + pos * 4) : 0x80000000u;
     };
     auto load_item = [&](int i, int c16, int p0) {
         const int e = tid + i * NT;
@@ -1394,13 +1394,15 @@ void split_gemm(GemmArgs g) {
                                xrs, static_cast<int>(strided_off(c16 * 16 + (e & 1) * 8 + j, pos)), 0, 0));
             return;
         }
-        // past the row: an offset past the buffer reads 0; so do channels past C_in
+        // past the row: an offset past the buffer reads 0; so do channels past
+        // C_in, held at 2^31 (rows of 2^27 bytes and more would wrap to the first)
         unsigned off = pos >= 0 && pos < g.L_in && e < 2 * span
-                           ? static_cast<unsigned>((c16 * 16 + (e & 1) * 8) * rowB + pos * 4) : 0x80000000u;
+                           ? static_cast<unsigned>(min(c16 * 16 + (e & 1) * 8, g.C_in) * rowB) + static_cast<unsigned>(pos) * 4u
+                           : 0x80000000u;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             xr[i][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrs, static_cast<int>(off), 0, 0));
-            off += rowB;
+            off = min(off + rowB, 0x80000000u);
         }
     };
     auto load_x = [&](int ch) {
@@ -1527,7 +1529,7 @@ void split_gemm(GemmArgs g) {
                         av[u] = weight(T.m0 + wm * 64 + u * 32 + l32, v, t);
                         const int pos = q - T.p;
                         const unsigned off = KT < 0 ? strided_off(v, q)
-                                             : pos >= 0 && pos < g.L_in ? static_cast<unsigned>(v * rowB + pos * 4)
+                                             : v < g.C_in && pos >= 0 && pos < g.L_in ? static_cast<unsigned>(v * rowB + pos * 4)
                                                                         : 0x80000000u;
                         bv[u] = __builtin_bit_cast(
                             float, __builtin_amdgcn_raw_buffer_load_b32(xrs, static_cast<int>(off), 0, 0));

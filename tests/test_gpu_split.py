@@ -256,3 +256,17 @@ def test_large_weights(K, kind):
         ref = torch.cat([w[m:m + 2048].double() @ dy.double().reshape(-1) for m in range(0, ci, 2048)])
     # 50 000 terms: sqrt(n) 2^-24
     assert rel(dx.reshape(-1), ref.cpu()) <= 1.4e-5
+
+
+def test_dgrad_rows_past_2_27_bytes(K):
+    # one channel of 2^28 positions: the chunk's other fifteen lie past the
+    # input and read zero, so an infinity reaches three results and makes no NaN
+    L, q = 1 << 28, 123_456_789
+    w, dy = torch.full((1, 3), 0.5, device="cuda"), torch.zeros(1, 1, L, device="cuda")
+    dy[0, 0, q] = float("inf")
+    dy[0, 0, 5] = 2.0
+    dx = torch.empty(1, 1, L, device="cuda")
+    K.call("kdec_conv1d_dgrad", P(w), P(dy), L, P(dx), L, 1, 1, L, 1, 3, 1, 1, 1, 1.0, 0.0)
+    assert torch.equal(dx[0, 0, q - 1:q + 2].cpu(), torch.full((3,), float("inf")))
+    assert torch.equal(dx[0, 0, 4:7].cpu(), torch.ones(3))
+    assert int(dx.count_nonzero()) == 6 and not bool(dx.isnan().any())
