@@ -2021,9 +2021,9 @@ struct WgradArgs {
     int M, C_x, L_x, L_g, k, s, p;
     // Column (c, t) as virtual channel v = c * R + r and tap q, t = q * R + r:
     // at position l it meets X[c][(l + q * sh) * s + r * rd - p].
-    //   stride 1          R = 1, T = k, sh = d
-    //   strided, d = 1    R = s, rd = 1, T = cdiv(k, s), sh = 1
-    //   strided, dilated  R = k, rd = d, T = 1
+    //   stride 1                             R = 1, T = k, sh = d
+    //   strided, d = 1                       R = min(s, k), rd = 1, T = cdiv(k, R), sh = 1
+    //   strided, dilated, and few channels   R = k, rd = d, T = 1
     int R, rd, T, sh;
     int NB;              // 32-column blocks: cdiv(C_x * R, 32) channel groups x T taps, tap fastest
     int chunks_per_n, total_chunks, splits;
@@ -3278,8 +3278,19 @@ static int wgrad_common(kdec_ctx* ctx, const float* X, long x_bs, const float* G
     WgradArgs a{};
     a.X = X; a.x_bs = x_bs; a.G = G; a.g_bs = g_bs;
     a.M = M; a.C_x = C_x; a.L_x = L_x; a.L_g = L_g; a.k = k; a.s = s; a.p = p;
-    const bool s1 = s == 1;
-    a.R = s1 ? 1 : d == 1 ? s : k;
+    // Groups of 32 channels by taps; or, of few channels and many taps, all taps
+    // as channels. Those columns are packed, but none share a window, and at
+    // stride 1 its loop runs at half the rate: taken from half as many tiles
+    // down, of one tile, or less than half. Taps / packed at M = 128, 8 x 61441:
+    // 1 channel, k = 11, 3 tiles / 1: 223 / 90 us; 8, k = 11, 3 / 1: 234 / 162;
+    // 16, k = 7, 2 / 1: 190 / 169; 22, k = 11, 3 / 2: 273 / 315; 33, k = 11,
+    // 6 / 3: 439 / 459.
+    a.R = s == 1 ? 1 : d == 1 ? std::min(s, k) : k;
+    auto tiles = [&](long R) { return cdiv(cdiv(C_x * R, 32) * cdiv(k, R), 4); };
+    const long packed_tiles = tiles(k);
+    const bool packed = 2 * packed_tiles <= tiles(a.R) - (packed_tiles > 1);
+    if (packed) a.R = k;
+    const bool s1 = s == 1 && !packed;
     a.rd = d;
     a.T = static_cast<int>(cdiv(k, a.R));
     a.sh = s1 ? d : 1;

@@ -81,6 +81,9 @@ def test_operands_past_bf16(K, value, where):
     (1, 50, 128, 700, 11, 1, 5), (2, 20, 22, 257, 7, 1, 1), (1, 130, 64, 95, 1, 1, 1), (1, 9, 9, 900, 5, 1, 90),
     (2, 22, 40, 601, 12, 6, 1), (1, 1, 1, 131, 3, 2, 1), (1, 18, 20, 300, 4, 3, 5), (1, 40, 12, 500, 2, 1, 33),
     (1, 64, 128, 50001, 3, 1, 1),
+    # few channels, all taps as channels; one channel more or one tap less, by taps
+    (2, 1, 130, 333, 11, 1, 3), (1, 8, 20, 97, 31, 1, 1), (2, 16, 40, 260, 7, 1, 40), (1, 17, 9, 260, 7, 1, 1),
+    (1, 1, 5, 401, 12, 2, 1), (1, 2, 3, 64, 2, 1, 1), (1, 40, 33, 130, 1, 3, 1), (1, 5, 7, 130, 2, 5, 1),
 ])
 def test_wgrad_edges(K, N, ci, co, L, k, s, d):
     # column blocks of 32 channels by a tap (shared and separate windows), row
