@@ -1067,9 +1067,10 @@ void corr_gemm(GemmArgs g) {
     const int c0 = sub * COLS;              // the block's first column in the tile
     if (T.q0 + c0 >= T.n_q) return;         // uniform per block
 
-    const int cg = G > 0 ? k : g.cg, no = G > 0 ? 2 : g.no;
-    const int span = COLS + (cg - 1) * d;   // staged positions
-    const int spanp = g.spanp;              // LDS row stride in positions (corr_stage)
+    const int cg = G > 0 ? k : g.cg, no = g.no;
+    const int de = min(d, COLS);            // a tap's shift in the staged window (corr_setup)
+    const int span = COLS + (cg - 1) * de;  // staged positions
+    const int spanp = g.spanp;              // LDS row stride in positions (corr_setup)
     const int bufsz = no * 2 * spanp;
     const __amdgpu_buffer_rsrc_t xrs = uniform_rsrc(g.X + static_cast<long>(T.b) * g.x_bs, g.C_in * g.L_in * 4);
     const int x0 = T.q0 + c0 - T.p;         // input position of the first column at tap 0
@@ -1078,13 +1079,19 @@ void corr_gemm(GemmArgs g) {
     // items e = tid + 256 i: octet half e % (2 no), position e / (2 no)
     const int hsh = no;
     const int nitems = span << hsh;
+    int po[CORR_ITEMS];  // an item's position in the input window
+#pragma unroll
+    for (int i = 0; i < CORR_ITEMS; ++i) {
+        const int w = (tid + i * NT) >> hsh;
+        po[i] = x0 + (d > COLS ? w / COLS * d + w % COLS : w);
+    }
     f32x4 xr[CORR_ITEMS];
     auto load_x = [&](int o, int t) {
 #pragma unroll
         for (int i = 0; i < CORR_ITEMS; ++i) {
             if (wave * 64 + i * NT >= nitems) continue;  // uniform
             const int e = tid + i * NT, h = e & (2 * no - 1);
-            const int pos = x0 + t * d + (e >> hsh);
+            const int pos = po[i] + t * d;
             // past the row: an offset past the buffer reads 0; so do channels past C_in
             unsigned off = pos >= 0 && pos < g.L_in ? static_cast<unsigned>((o * 8 + h * 4) * rowB + pos * 4) : 0x80000000u;
 #pragma unroll
@@ -1148,8 +1155,8 @@ void corr_gemm(GemmArgs g) {
                     acc[0][tn] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[e], b[tn][e], acc[0][tn], 0, 0, 0);
         };
         if constexpr (G > 0) {
-            // chunks of two octets, all taps; the plan's chunks (up to G taps
-            // of an octet) unrolled, their weights one plan chunk ahead, the
+            // chunks of all taps; the plan's chunks (up to G taps of an octet)
+            // unrolled, their weights one plan chunk ahead, the
             // input a step ahead
             int w = p * nchunks / nparts, we = (p + 1) * nchunks / nparts;
             const int w1 = pb * nchunks / nparts;
@@ -1171,18 +1178,18 @@ void corr_gemm(GemmArgs g) {
             }
             store_x(0);
             __syncthreads();
-            if ((w1 - 1) / g.n_tg >= co + 2) load_x(co + 2, 0);
+            if ((w1 - 1) / g.n_tg >= co + no) load_x(co + no, 0);
             int buf = 0;
             for (; w < w1; ++w) {
                 const int gt = min(G, k - tg * G);
                 const int sn = min(s + gt, last);
                 const __amdgpu_buffer_rsrc_t ars = panel(sn);
-                const f32x4* row = lds + buf * bufsz + ((o - co) * 2 + hi) * spanp + l32 + tg * G * d;
+                const f32x4* row = lds + buf * bufsz + ((o - co) * 2 + hi) * spanp + l32 + tg * G * de;
                 f32x4 b[2][TN];
                 load_b(row, b[0]);
 #pragma unroll
                 for (int u = 0; u < G; ++u) {
-                    if (u + 1 < G) load_b(row + (u + 1 < gt ? u + 1 : 0) * d, b[(u + 1) & 1]);
+                    if (u + 1 < G) load_b(row + (u + 1 < gt ? u + 1 : 0) * de, b[(u + 1) & 1]);
                     if (u == 0 || u < gt) mma(ring[u], b[u & 1]);  // uniform
                     load_ring(sn, u, ars);
                     __builtin_amdgcn_sched_barrier(0);  // nothing crosses into the next step
@@ -1194,12 +1201,12 @@ void corr_gemm(GemmArgs g) {
                 }
                 if (++tg == g.n_tg) {
                     tg = 0;
-                    if (++o == co + 2 && w + 1 < w1) {
+                    if (++o == co + no && w + 1 < w1) {
                         co = o;
                         buf ^= 1;
                         store_x(buf);
                         __syncthreads();
-                        if ((w1 - 1) / g.n_tg >= co + 2) load_x(co + 2, 0);
+                        if ((w1 - 1) / g.n_tg >= co + no) load_x(co + no, 0);
                     }
                 }
             }
@@ -1223,7 +1230,7 @@ void corr_gemm(GemmArgs g) {
             for (int u = 0; u < D; ++u) ring[u] = load_a(s + u);
             store_x(0);
             __syncthreads();
-            int bo = hi * spanp + l32 + (t - ct) * d;
+            int bo = hi * spanp + l32 + (t - ct) * de;
             next(co, ct);
             if (ce < s1) load_x(co, ct);
             int buf = 0;
@@ -1236,10 +1243,10 @@ void corr_gemm(GemmArgs g) {
                     mma(ring[u], b);
                     ring[u] = load_a(s + D);
                     ++s;
-                    bo += d;
+                    bo += de;
                     if (++t == k) {  // the next octet's half rows
                         t = 0;
-                        bo += 2 * spanp - k * d;
+                        bo += 2 * spanp - k * de;
                     }
                     if (s == pe) fold();
                     if (s == ce && s < s1) {
@@ -2747,18 +2754,27 @@ const void* corr_kernel() {
     return reinterpret_cast<const void*>(&corr_gemm<G, TN>);
 }
 
+// Positions corr_gemm stages for `cols` columns of k taps.
+long corr_window(int cols, int k, int d) { return cols + (k - 1L) * std::min(d, cols); }
+
 // The corr_gemm instance for k taps at dilation d and blocks of `cols`
-// columns, and its staging: two octets with the window of all taps where
-// CORR_ITEMS items per thread hold it (with k >= 3, the plan chunks unrolled),
-// else one octet with as many taps as they do.
+// columns, and its staging: two octets, or one, with the window of all taps
+// where CORR_ITEMS items per thread hold it (with k >= 3, the plan chunks
+// unrolled), else one octet with as many taps as they do. Taps further apart
+// than the block's columns are staged by themselves, without the positions
+// between. 256 channels, L = 4000: k = 5, d = 200, 83 us with the positions
+// between and taps in groups, 46 here; k = 3, d = 300, 66 and 27; k = 7, d =
+// 100, 96 and 52.
 const void* corr_setup(GemmArgs& g, int cols, int k, int d) {
     const long most = CORR_ITEMS * NT;
-    const bool all = 4 * (cols + static_cast<long>(k - 1) * d) <= most;
-    g.no = all ? 2 : 1;
-    g.cg = all ? k : static_cast<int>(std::min(static_cast<long>(k), (most / 2 - cols) / d + 1L));
+    const int de = std::min(d, cols);
+    const long window = corr_window(cols, k, d);
+    const bool all = 2 * window <= most;
+    g.no = 4 * window <= most ? 2 : 1;
+    g.cg = all ? k : static_cast<int>((most / 2 - cols) / de + 1L);
     // 4 / no mod 16: the staging stores of 2 no octet halves by 4 / no
     // positions spread over the banks
-    const int sp = cols + (g.cg - 1) * d, want = 4 / g.no;
+    const int sp = cols + (g.cg - 1) * de, want = 4 / g.no;
     g.spanp = sp + ((want - sp % 16) + 16) % 16;
     if (all && g.G == 3) return cols == 64 ? corr_kernel<3, 2>() : corr_kernel<3, 1>();
     if (all && g.G == 4) return cols == 64 ? corr_kernel<4, 2>() : corr_kernel<4, 1>();
@@ -2906,7 +2922,9 @@ int run_gemm(kdec_ctx* ctx, GemmArgs g, int N, int m_tiles, const char* fam,
         // CUs (376 tiles of 352 steps: 270 us, with 32 columns 285; 126 tiles
         // of 224 steps: 81, with 32 columns 77)
         const long bt = g.serial ? tiles : tiles * f;
-        const int cols = max_q > 32 && bt * 4 >= 5L * ctx->num_cus ? 64 : 32;
+        int cols = max_q > 32 && bt * 4 >= 5L * ctx->num_cus ? 64 : 32;
+        // (32 where only they hold all taps: 256 channels, L = 4000, k = 11, d = 33: 84 us with 64, 74)
+        if (2 * corr_window(64, kk, dd) > CORR_ITEMS * NT && 2 * corr_window(32, kk, dd) <= CORR_ITEMS * NT) cols = 32;
         kern = corr_setup(g, cols, kk, dd);
         lds = 2 * 2 * static_cast<size_t>(g.no) * g.spanp * 16;
         g.nsub = static_cast<int>(cdiv(std::min(max_q, BN), cols));

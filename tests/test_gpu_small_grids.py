@@ -36,7 +36,12 @@ TOL = 3.5e-6
     (1, 128, 22, 24121, 7, 1),
     (1, 64, 40, 3000, 2, 1), (1, 24, 40, 3000, 5, 1), (1, 200, 512, 400, 1, 1),
     (1, 32, 64, 2000, 5, 60),      # a window past the staging items: taps in groups
-    (1, 32, 64, 2000, 3, 300),     # one tap at a time
+    (1, 32, 64, 2000, 3, 300),     # taps further apart than the block's columns
+    (1, 40, 64, 2000, 5, 200), (4, 32, 64, 20000, 5, 200),  # those in blocks of 32 and of 64 columns, all at once
+    (1, 40, 64, 2000, 7, 100), (1, 24, 130, 400, 11, 33), (4, 24, 64, 20000, 7, 33),  # an octet's at once
+    (4, 24, 64, 20000, 9, 70), (1, 72, 40, 1500, 20, 40),   # and in groups
+    (1, 32, 64, 2000, 3, 32), (1, 32, 64, 2000, 3, 33), (4, 24, 64, 20000, 3, 64), (4, 24, 64, 20000, 3, 65),
+    (1, 9, 17, 1500, 2, 500), (1, 16, 130, 33, 3, 90),
 ])
 def test_conv_fwd_edges(K, N, ci, co, L, k, d):
     g = torch.Generator().manual_seed(ci + L)
