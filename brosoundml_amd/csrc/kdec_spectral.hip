@@ -1294,10 +1294,16 @@ int kdec_style_proj_bwd(kdec_ctx* ctx, const float* W, const float* style,
         if (int rc = launch_check(ctx, "style_bwd_x_reduce")) return rc;
     }
     // the row kernel where a row's quads divide a block, dW takes 16-byte
-    // accesses and the operands of all utterances fit 48 KB of LDS
+    // accesses, the operands of all utterances fit 48 KB of LDS, and there are
+    // enough blocks to cover the wait for those operands, which a thread per
+    // element does not have: half a round and one for each 16 of them (measured
+    // element / row: N = 8, S = 128, 128 blocks 5.5 / 5.6 us, 256 7.8 / 5.9;
+    // N = 24, S = 128, 160 blocks 9.7 / 10.3, 256 12.1 / 10.6; N = 8, S = 1024,
+    // 400 blocks 9.3 / 12.0, 800 15.7 / 14.6)
     const long wrows = S > 0 && S % 4 == 0 ? SWR * (1024L / S) : 0;
     const long wlds = static_cast<long>(N) * (S + wrows) * static_cast<long>(sizeof(float));
-    if (dW && wrows > 0 && 1024 % S == 0 && wlds <= 48 * 1024 && (reinterpret_cast<unsigned long long>(dW) & 15) == 0) {
+    const bool wfill = wrows > 0 && 16 * (cdiv(rows, wrows) - ctx->num_cus / 2) >= wlds / 4;
+    if (dW && wfill && 1024 % S == 0 && wlds <= 48 * 1024 && (reinterpret_cast<unsigned long long>(dW) & 15) == 0) {
         hipLaunchKernelGGL(style_bwd_w_rows_k, dim3(static_cast<unsigned>(cdiv(rows, wrows))), dim3(256),
                            static_cast<size_t>(wlds), ctx->stream, style, style_bs, dout, dout_bs, dW, db, N, rows, S);
         if (int rc = launch_check(ctx, "style_bwd_w_rows")) return rc;

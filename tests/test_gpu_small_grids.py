@@ -67,7 +67,11 @@ def test_convt_fwd_edges(K, k, s, L):
     assert rel(y, F.conv_transpose1d(x.double(), w.double().reshape(ci, co, k), stride=s, padding=p)) <= TOL
 
 
-@pytest.mark.parametrize("N,rows,S", [(1, 1, 128), (8, 33, 128), (9, 100, 64), (40, 17, 256), (3, 31, 4), (80, 20, 128)])
+@pytest.mark.parametrize("N,rows,S", [(1, 1, 128), (8, 33, 128), (9, 100, 64), (40, 17, 256), (3, 31, 4), (80, 20, 128),
+                                      # above, an element per thread; from 208 blocks of 32 rows on (N = 8,
+                                      # S = 128) by rows: whole blocks, a part of the last, one block less
+                                      (8, 6656, 128), (8, 6655, 128), (8, 6624, 128), (9, 17471, 64), (1, 8900, 64),
+                                      (3, 3195, 256), (1, 197700, 4), (1, 803, 1024), (1, 803, 1022)])
 def test_style_weight_grad(K, N, rows, S):
     g = torch.Generator().manual_seed(N)
     st, do = torch.randn(N, S, generator=g), torch.randn(N, rows, generator=g)
