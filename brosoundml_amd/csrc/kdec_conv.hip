@@ -1966,46 +1966,110 @@ __global__ void pack_octet(const float* W, float* A, int mode, int C_in, int C_o
     }
 }
 
-// split_gemm's weight panel [m_tile][step = c16*k + t][plane][32-row block]
-// [lane][8] of a conv1d input-grad (s = 0), A[(co, t), ci] = W[co, ci*k + k-1-t],
-// or of a transposed conv's at stride s, kt = cdiv(k, s) taps, channel (co, r <
-// R = min(s, k)): A[(co, r, t), ci] = W[ci, co*k + t*s + r], zero where that is past k. Lane
-// (hi, l32) of block mb holds row ci = 32 mb + l32 of the tile, channels co =
-// 16 c16 + 8 hi + j, split in three bf16 planes; zero past either. One thread
-// per (step, block, lane).
-__global__ void pack_split(const float* W, float* A, int C_in, int C_out, int k, int s, int R, int kt,
-                           int nsteps, long total) {
-    for (long i = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x; i < total;
-         i += static_cast<long>(gridDim.x) * blockDim.x) {
-        const unsigned iu = static_cast<unsigned>(i);  // total < 2^31: a 12th of the panel's floats (the host's checks)
-        const int lane = iu & 63, mb = (iu >> 6) & 3;
-        const unsigned rest = iu >> 8;
-        const unsigned st = rest % static_cast<unsigned>(nsteps);
-        const int mt = static_cast<int>(rest / static_cast<unsigned>(nsteps));
-        const int c16 = static_cast<int>(st) / kt, t = static_cast<int>(st) - c16 * kt;
-        const int m = mt * BM + mb * 32 + (lane & 31);
-        const int c0 = c16 * 16 + (lane >> 5) * 8;
-        float v[8];
+// split_gemm's weight panel [m_tile][step = c16*kt + t][plane][32-row block]
+// [lane][8]: of a conv1d input-grad (TR = false, kt = k) A[(co, t), ci] =
+// W[co, ci*k + k-1-t], of a transposed conv's at stride s, kt = cdiv(k, s)
+// taps, channel (co, r < R = min(s, k)), A[(co, r, t), ci] = W[ci, co*k + t*s +
+// r], zero where that is past k. Lane (hi, l32) of block mb holds row ci = 32 mb
+// + l32 of the tile, channels 16 c16 + 8 hi + j, split in three bf16 planes;
+// zero past either.
+//
+// A block packs 16 channels of nmb 32-row blocks. Bound by HBM: the weights are
+// read in their own order (a channel's run of 32 nmb rows by k taps, at most gt
+// of them at a time; a row's run of the 16 channels by k) into LDS, from where a
+// wave takes one tap of a 32-row block. With a thread per lane of a fragment,
+// eight loads k floats apart from its neighbours' each, 2048 x 2048 weights of
+// 11 taps took 228 us (2.0 TB/s read and written), 78 here; 512 x 512 of 7, 11
+// and 8. 128 x 128 of 11 take 4.6 us for 3.6: few blocks.
+struct PackSplit {
+    const float* W;
+    float* A;
+    int C_in, C_out, k, s, R, kt;
+    int n_c16, mblocks;  // channel chunks; blocks of nmb 32-row blocks
+    int nmb, gt;
+};
+
+template <bool TR>
+__global__ __launch_bounds__(256) void pack_split(PackSplit g) {
+    extern __shared__ float wt[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l32 = lane & 31, hi = lane >> 5;
+    // channel chunks fastest: neighbouring blocks write neighbouring steps (1024 x
+    // 1024, k = 3: 13.7 us with row blocks fastest, 9.8 so, 10.0 a thread per lane)
+    const int c16 = static_cast<int>(blockIdx.x % static_cast<unsigned>(g.n_c16));
+    const int rest = static_cast<int>(blockIdx.x / static_cast<unsigned>(g.n_c16));
+    const int mb0 = rest % g.mblocks * g.nmb, k0 = rest / g.mblocks * g.gt;
+    const int m0 = mb0 * 32, k = g.k;
+    const int taps = TR ? g.kt : min(g.gt, k - k0);  // stored taps k0 .. k0 + taps - 1 (TR: all kt)
+    int rs;           // LDS row stride
+    int at[8];        // TR: offsets in a row of the lane's channels at tap 0, and their phases
+    int ph[8];
+    if constexpr (TR) {
+        const int v0 = c16 * 16, lo = v0 / g.R;
+        const int run = (min((v0 + 15) / g.R, g.C_out - 1) - lo + 1) * k;
+        rs = run | 1;
+        const int rows = 32 * g.nmb;
+        for (int e = lane; e < run; e += 64)
+            for (int r0 = wave; r0 < rows; r0 += 32) {
+                float x[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const int m = m0 + r0 + 4 * u;
+                    x[u] = m < g.C_in ? g.W[(static_cast<long>(m) * g.C_out + lo) * k + e] : 0.0f;
+                }
+#pragma unroll
+                for (int u = 0; u < 8; ++u) wt[(r0 + 4 * u) * rs + e] = x[u];
+            }
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            const int c = c0 + j;
-            if (s == 0) {
-                v[j] = m < C_in && c < C_out ? W[(static_cast<long>(c) * C_in + m) * k + (k - 1 - t)] : 0.0f;
-            } else {
-                const int co = c / R, tt = t * s + c - co * R;
-                v[j] = m < C_in && co < C_out && tt < k ? W[(static_cast<long>(m) * C_out + co) * k + tt] : 0.0f;
-            }
+            const int v = v0 + hi * 8 + j, c = v / g.R;
+            ph[j] = c < g.C_out ? v - c * g.R : k;  // past the channels: past every tap
+            at[j] = (c - lo) * k + ph[j];
         }
+    } else {
+        const int run = 32 * g.nmb * taps;
+        rs = run + 4;  // the halves' channels, eight rows apart, half the banks apart
+        for (int e0 = lane; e0 < run; e0 += 128) {  // wave w: channels 4w .. 4w + 3
+            float x[2][4];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int e = e0 + 64 * h;
+                const int m = taps == k ? 0 : e / taps;
+                const int o = taps == k ? e : m * k + k0 + e - m * taps;  // within the channel's run
+                const bool in = e < run && static_cast<long>(m0) * k + o < static_cast<long>(g.C_in) * k;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int c = c16 * 16 + wave * 4 + u;
+                    x[h][u] = in && c < g.C_out ? g.W[(static_cast<long>(c) * g.C_in + m0) * k + o] : 0.0f;
+                }
+            }
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (e0 + 64 * h < run) wt[(wave * 4 + u) * rs + e0 + 64 * h] = x[h][u];
+        }
+    }
+    __syncthreads();
+    for (int i = wave; i < g.nmb * taps; i += 4) {
+        const int mb = i % g.nmb, u = i / g.nmb;
         bf16x8 p[3];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
+            float v;
+            if constexpr (TR)
+                v = u * g.s + ph[j] < k ? wt[(mb * 32 + l32) * rs + at[j] + u * g.s] : 0.0f;
+            else
+                v = wt[(hi * 8 + j) * rs + (mb * 32 + l32) * taps + u];
             __bf16 h, q, l;
-            split3(v[j], h, q, l);
+            split3(v, h, q, l);
             p[0][j] = h;
             p[1][j] = q;
             p[2][j] = l;
         }
-        float* o = A + static_cast<long>(rest) * SPLIT_STEP + mb * 256 + lane * 4;
+        const int t = TR ? u : k - 1 - (k0 + u);
+        const long step = static_cast<long>((mb0 + mb) >> 2) * g.n_c16 * g.kt + static_cast<long>(c16) * g.kt + t;
+        float* o = g.A + step * SPLIT_STEP + ((mb0 + mb) & 3) * 256 + lane * 4;
 #pragma unroll
         for (int pl = 0; pl < 3; ++pl) *reinterpret_cast<bf16x8*>(o + pl * 1024) = p[pl];
     }
@@ -2831,6 +2895,48 @@ void split_setup(GemmArgs& g, int C, int k, int d) {
 // Floats of split_gemm's weight panel for M output rows.
 long split_panel(const GemmArgs& g, int M) { return cdiv(M, BM) * g.n_c16 * g.k * SPLIT_STEP; }
 
+template <bool TR>
+const void* pack_split_kernel() {
+    static bool attr = false;
+    if (!attr) {
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&pack_split<TR>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        attr = true;
+    }
+    return reinterpret_cast<const void*>(&pack_split<TR>);
+}
+
+// Packs split_gemm's panel of the weights to M rows: of a conv's input grad (wk =
+// 0, C channels) or a transposed conv's (wk taps, C * nph channels).
+int launch_pack_split(kdec_ctx* ctx, const GemmArgs& g, float* A, int M, int C, const char* what) {
+    const bool tr = g.wk > 0;
+    PackSplit a{};
+    a.W = g.W;
+    a.A = A;
+    a.C_in = M;
+    a.C_out = C;
+    a.k = tr ? g.wk : g.k;
+    a.s = g.s;
+    a.R = tr ? g.nph : 1;
+    a.kt = g.k;
+    a.n_c16 = g.n_c16;
+    a.gt = tr ? a.k : std::min(a.k, 31);  // (64 KB; a transposed conv has k <= 32)
+    // more 32-row blocks where one is less than 64 floats of a channel
+    const long run = tr ? std::min(static_cast<long>(C), (14L + a.R) / a.R + 1) * a.k : 32L * a.gt;
+    auto bytes = [&](int nmb) { return (tr ? 32L * nmb * (run | 1) : 16L * (nmb * run + 4)) * 4; };
+    a.nmb = tr || a.k > 2 ? 1 : a.k == 2 ? 2 : 4;
+    const long m_blocks = cdiv(M, BM) * (4 / a.nmb);
+    const long blocks = m_blocks * a.n_c16 * (tr ? 1 : cdiv(a.k, a.gt));
+    if (blocks > 0x7fffffffL) return fail(ctx, KDEC_EINVAL, "conv: weights too large");
+    a.mblocks = static_cast<int>(m_blocks);
+    void* args[] = {&a};
+    const void* kern = tr ? pack_split_kernel<true>() : pack_split_kernel<false>();
+    if (hipLaunchKernel(kern, dim3(static_cast<unsigned>(blocks)), dim3(256), args, static_cast<size_t>(bytes(a.nmb)),
+                        ctx->stream) != hipSuccess)
+        return fail(ctx, KDEC_EHIP, std::string(what) + ": launch failed");
+    return launch_check(ctx, what);
+}
+
 // Launches a GEMM kernel over an already packed A.
 //
 // Work plan: with S resident blocks, T tiles take T / S whole rounds plus a
@@ -3191,10 +3297,7 @@ int conv_dgrad_impl(kdec_ctx* ctx, const float* W, const float* dY, long dy_bs, 
     Workspace A(ctx, static_cast<size_t>(tot) * sizeof(float));
     if (!A.p) return KDEC_ENOMEM;
     g.A = A.as<float>();
-    const long items = tot / SPLIT_STEP * 256;
-    hipLaunchKernelGGL(pack_split, dim3(grid1d(items)), dim3(256), 0, ctx->stream, W, A.as<float>(), C_in, C_out, k,
-                       0, 1, k, g.n_c16 * k, items);
-    if (int rc = launch_check(ctx, "pack_dgrad")) return rc;
+    if (int rc = launch_pack_split(ctx, g, A.as<float>(), C_in, C_out, "pack_dgrad")) return rc;
     return run_gemm(ctx, g, N, m_pad / BM, "conv_dgrad",
                     2.0 * N * C_out * static_cast<double>(L_out) * C_in * k);
 }
@@ -3494,13 +3597,8 @@ int kdec_convt1d_dgrad(kdec_ctx* ctx, const float* W, const float* dY,
     KDEC_CHECK(ctx, static_cast<long>(C_out) * g.nph <= 0x7fffffffL - 16, "kdec_convt1d_dgrad: weights too large");
     split_setup(g, C_out * g.nph, g.k, 1);
     const long tot = split_panel(g, C_in);
-    KDEC_CHECK(ctx, tot / 12 <= 0x7fffffffL, "kdec_convt1d_dgrad: weights too large");  // pack_split's items
     Workspace A(ctx, static_cast<size_t>(tot) * sizeof(float));
     if (!A.p) return KDEC_ENOMEM;
-    const long items = tot / SPLIT_STEP * 256;
-    hipLaunchKernelGGL(pack_split, dim3(grid1d(items)), dim3(256), 0, ctx->stream, W, A.as<float>(), C_in, C_out, k,
-                       stride, g.nph, g.k, g.n_c16 * g.k, items);
-    if (int rc = launch_check(ctx, "pack_convt_dgrad")) return rc;
     const int m_pad = static_cast<int>(cdiv(C_in, BM) * BM);
     g.X = dY; g.x_bs = dy_bs; g.A = A.as<float>();
     g.Y = dX; g.y_bs = dx_bs;
@@ -3510,6 +3608,7 @@ int kdec_convt1d_dgrad(kdec_ctx* ctx, const float* W, const float* dY,
     g.scale = 1.0f; g.beta = 0.0f; g.n_phase = 1;
     g.W = W;
     g.wk = k;
+    if (int rc = launch_pack_split(ctx, g, A.as<float>(), C_in, C_out, "pack_convt_dgrad")) return rc;
     return run_gemm(ctx, g, N, m_pad / BM, "convt_dgrad",
                     2.0 * N * C_in * static_cast<double>(L) * C_out * k);
 }

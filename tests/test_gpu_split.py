@@ -34,6 +34,7 @@ TOL = 2.5e-6
     (1, 1, 1, 1, 1, 1), (2, 127, 15, 127, 3, 1), (1, 128, 16, 128, 7, 3), (3, 129, 17, 129, 11, 5),
     (1, 128, 22, 401, 7, 1), (2, 128, 128, 1001, 11, 1), (1, 130, 40, 300, 11, 13), (1, 20, 20, 1500, 5, 200),
     (2, 22, 128, 257, 1, 1), (1, 1090, 64, 31, 3, 1), (1, 64, 128, 40000, 2, 9),
+    (1, 35, 3, 200, 33, 1), (1, 5, 18, 300, 70, 1),  # weights packed in more than one group of taps
 ])
 def test_dgrad_edges(K, N, ci, co, L, k, d):
     g = torch.Generator().manual_seed(ci * 1000 + L)
@@ -137,6 +138,7 @@ def test_wgrad_operands_past_bf16(K, value, where):
 @pytest.mark.parametrize("N,ci,co,k,s,L", [
     (2, 130, 24, 20, 10, 33), (1, 127, 17, 12, 6, 130), (1, 9, 1, 3, 4, 9), (2, 20, 40, 5, 1, 140), (1, 64, 3, 7, 3, 257),
     (1, 30, 33, 1, 8, 260), (2, 9, 5, 3, 10, 40), (1, 130, 16, 7, 8, 31),
+    (1, 40, 20, 32, 1, 90), (1, 33, 20, 32, 16, 9),
 ])
 def test_convt_dgrad_edges(K, N, ci, co, k, s, L):
     # a stride's phases as channels: k a multiple of the stride and not, fewer
