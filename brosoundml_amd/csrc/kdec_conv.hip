@@ -3003,8 +3003,11 @@ int run_gemm(kdec_ctx* ctx, GemmArgs g, int N, int m_tiles, const char* fam,
     // and reduction cost more than the idle slots (128 channels, k = 3, 2 x 7681,
     // 120 tiles of 24 steps: 34 us in parts, 26 whole; k = 7, 24121, 189 of 56:
     // 53 / 43; k = 11, 2 x 7681, 120 of 88: 49 / 55; 256 channels, k = 7, 4000,
-    // 64 of 112: 40 / 46 in two)
-    const bool whole = split && 2L * g.n_c16 * kk * ctx->num_cus <= tiles * 256;
+    // 64 of 112: 40 / 46 in two). Past the first round the last one's tiles do,
+    // unless an eighth of a round or less (512 slots, parts / whole: 128
+    // channels, k = 11, 520 tiles of 88 steps 125 / 150, 576 140 / 151, 640 156 /
+    // 153, 768 177 / 167; k = 3, 576 of 24 54 / 58, 640 62 / 59)
+    const bool whole = split && (tiles > slots ? 8 * rem > slots : 2L * g.n_c16 * kk * ctx->num_cus <= tiles * 256);
     if (rem > 0 && !whole) f = std::min(std::min(slots / rem, parts), 16L);
     if (f < 2) f = 1;
     g.fsplit = static_cast<int>(f);

@@ -55,6 +55,22 @@ def test_conv_fwd_edges(K, N, ci, co, L, k, d):
     assert rel(y, 0.5 * (ref + r.double()) + 2.0 * y0.double()) <= TOL
 
 
+def test_conv_fwd_parts(K):
+    # 64 tiles of 384 steps: in parts, a block each, summed by tile_reduce
+    N, ci, co, L, k, p = 8, 1024, 1000, 100, 3, 1
+    g = torch.Generator().manual_seed(1)
+    x, w, b, r, y0 = (torch.randn(*s, generator=g) for s in ((N, ci, L), (co, ci * k), (co,), (N, co, L), (N, co, L)))
+    xg, wg, bg, rg, y = x.cuda(), w.cuda(), b.cuda(), r.cuda(), y0.cuda()
+    K.profile(True)
+    K.profile_reset()
+    K.call("kdec_conv1d_fwd", P(xg), ci * L, P(wg), P(bg), P(y), co * L, N, ci, L, co, k, 1, p, 1, P(rg), co * L, 0.5, 2.0)
+    torch.cuda.synchronize()
+    assert "tile_reduce" in K.profile_read()
+    K.profile(False)
+    ref = F.conv1d(x.double(), w.double().reshape(co, ci, k), b.double(), padding=p)
+    assert rel(y, 0.5 * (ref + r.double()) + 2.0 * y0.double()) <= TOL
+
+
 @pytest.mark.parametrize("k,s,L", [(20, 10, 42), (20, 10, 400), (12, 6, 4000), (3, 4, 9), (5, 1, 140)])
 def test_convt_fwd_edges(K, k, s, L):
     N, ci, co, p = 1, 72, 136, max(0, (k - s) // 2)

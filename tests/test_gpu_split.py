@@ -275,3 +275,69 @@ def test_dgrad_rows_past_2_27_bytes(K):
     assert torch.equal(dx[0, 0, q - 1:q + 2].cpu(), torch.full((3,), float("inf")))
     assert torch.equal(dx[0, 0, 4:7].cpu(), torch.ones(3))
     assert int(dx.count_nonzero()) == 6 and not bool(dx.isnan().any())
+
+
+def families(K, f):
+    """The profile's kernel families of one call."""
+    K.profile(True)
+    K.profile_reset()
+    f()
+    torch.cuda.synchronize()
+    names = set(K.profile_read())
+    K.profile(False)
+    return names
+
+
+@pytest.mark.parametrize("N,ci,co,L,k,d", [
+    (1, 128, 128, 128 * 520 - 5, 3, 1),  # a round of whole tiles, eight in parts
+    (259, 130, 96, 20, 31, 1),           # 518 tiles, 31 taps in parts that end between them
+    (8, 1024, 1024, 100, 3, 1),          # less than a round, all in parts
+    (1, 300, 260, 31, 11, 13),           # two tap groups per chunk
+])
+def test_dgrad_parts(K, N, ci, co, L, k, d):
+    # tiles in parts (the profile shows their reduction), with whole ones and
+    # without; dX = scale * sums + beta * dX
+    g = torch.Generator().manual_seed(L)
+    p = d * (k - 1) // 2
+    w, dy, dx0 = (torch.randn(*s, generator=g) for s in ((co, ci * k), (N, co, L), (N, ci, L)))
+    wg, dyg, dx = w.cuda(), dy.cuda(), dx0.cuda()
+    f = lambda: K.call("kdec_conv1d_dgrad", P(wg), P(dyg), co * L, P(dx), ci * L, N, ci, L, co, k, 1, p, d, 0.5, 2.0)
+    assert "tile_reduce" in families(K, f)
+    ref = F.conv_transpose1d(dy.double(), w.double().reshape(co, ci, k), padding=p, dilation=d)
+    # up to 3072 terms: sqrt(n) 2^-24
+    assert rel(dx, 0.5 * ref + 2.0 * dx0.double()) <= 3.4e-6
+
+
+@pytest.mark.parametrize("N,C,Co,L,k,d,act,with_r,parts", [
+    (515, 256, 128, 20, 5, 1, 1, True, True),    # 1030 tiles, six in parts; taps at run time
+    (515, 200, 128, 20, 3, 1, 2, True, True),    # a partial row tile, Snake
+    (129, 128, 48, 1001, 11, 5, 2, False, True),  # 1032 tiles over row ends
+    (515, 256, 96, 20, 5, 40, 0, False, True),   # tap groups
+    (600, 256, 64, 20, 5, 1, 1, True, False),    # 1200 tiles, all whole
+    (1024, 40, 20, 9, 1, 1, 2, True, False), (8, 128, 32, 128 * 128, 7, 1, 1, False, False),
+])
+def test_dgrad_adain_bwd_parts(K, N, C, Co, L, k, d, act, with_r, parts):
+    # the AdaIN backward in the GEMM's epilogue and in the parts' reduction,
+    # against the two calls the one replaces
+    g = torch.Generator(device="cuda").manual_seed(C + L)
+    rn = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    p = d * (k - 1) // 2
+    x, w, dy, r = rn(N, C, L) + 0.2, rn(Co, C * k) / (C * k) ** 0.5, rn(N, Co, L), rn(N, C, L)
+    gm, bt, al = rn(N, C) * 0.4, rn(N, C) * 0.3, torch.rand(C, generator=g, device="cuda") + 0.5
+    st, da0 = torch.empty(N * C, 2, device="cuda"), rn(C)
+    K.call("kdec_instnorm_stats", P(x), C * L, N, C, L, 1e-5, P(st))
+    R = P(r) if with_r else None
+    got, ref = ([torch.empty(N, C, L, device="cuda"), torch.empty(N, C, device="cuda"), torch.empty(N, C, device="cuda"),
+                 da0.clone()] for _ in range(2))
+    out = lambda o: (P(o[0]), C * L, P(o[1]), P(o[2]), C, P(o[3]))
+    fam = families(K, lambda: K.call(
+        "kdec_conv1d_dgrad_adain_bwd", P(w), P(dy), Co * L, N, C, L, Co, k, 1, p, d, P(x), C * L, P(st), P(gm), P(bt), C,
+        act, 0.2, P(al), R, C * L, *out(got)))
+    assert ("tile_reduce" in fam) == parts
+    t = torch.empty(N, C, L, device="cuda")
+    K.call("kdec_conv1d_dgrad", P(w), P(dy), Co * L, P(t), C * L, N, C, L, Co, k, 1, p, d, 1.0, 0.0)
+    K.call("kdec_adain_act_bwd", P(x), C * L, P(st), P(gm), P(bt), C, act, 0.2, P(al), P(t), C * L, R, C * L, *out(ref),
+           N, C, L)
+    # the same sums in another order: the row sums (L terms) and dalpha (N L terms) in double
+    for a, b in zip(got, ref):
+        assert rel(a, b.double().cpu()) <= 2e-6
