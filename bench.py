@@ -32,6 +32,9 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 PEAK_FP32_MFMA = 157.3e12   # MI355X dense FP32 matrix, FLOP/s
+# Float multiply-adds of the split grads, six bf16 products each: MI355X's
+# dense bf16 matrix peak, 2.5 PFLOP/s, over six.
+PEAK_SPLIT_MFMA = 2.5e15 / 6
 PEAK_HBM = 8.0e12           # MI355X HBM3E, B/s
 B, T = 8, 512
 
@@ -303,7 +306,7 @@ def micro_benches(ctx, reps=50):
         tot_f += 2 * 2.0 * N * C * C * k * L
     out["conv1d_bwd_512x512_k3_d135_x4x2048"] = {"ms": round(tot_t * 1e3, 4),
                                                  "TFLOP/s": round(tot_f / tot_t / 1e12, 2),
-                                                 "frac_mfma": round(tot_f / tot_t / PEAK_FP32_MFMA, 4),
+                                                 "frac_mfma": round(tot_f / tot_t / PEAK_SPLIT_MFMA, 4),
                                                  "flop": tot_f}
     del X, G, W, dX, dW
 
@@ -326,7 +329,7 @@ def micro_benches(ctx, reps=50):
         t = timed(run)
         fl = 2 * 2.0 * 4 * Ci * Co * kk * Lin
         res[name] = {"ms": round(t * 1e3, 4), "TFLOP/s": round(fl / t / 1e12, 2),
-                     "frac_mfma": round(fl / t / PEAK_FP32_MFMA, 4), "flop": fl}
+                     "frac_mfma": round(fl / t / PEAK_SPLIT_MFMA, 4), "flop": fl}
     out["convT_bwd"] = res
     del Xt, Gt, Wt, dXt, dWt
 
@@ -516,8 +519,22 @@ def main(argv=None):
     audio_per_step = B * lens["audio_seconds"]
     value = audio_per_step / (dt / a.steps)
 
-    # dominant kernel: the conv implicit GEMM family with the most time
-    GEMM_FAMS = ("conv_fwd", "conv_dgrad", "convt_fwd", "convt_dgrad")
+    # dominant kernel: the forward convs' GEMMs, on the FP32 matrix unit; the
+    # input and weight grads' are split ones on the bf16 unit, each priced at
+    # its own unit's rate
+    GEMM_FAMS = ("conv_fwd", "convt_fwd")
+    GRAD_FAMS = {"dgrad_roofline": ("split_gemm (conv1d and convT input grads)", ("conv_dgrad", "convt_dgrad")),
+                 "wgrad_roofline": ("wgrad_gemm", ("conv_wgrad", "convt_wgrad"))}
+
+    def grad_roofline(prof, key, n):
+        kernel, fams = GRAD_FAMS[key]
+        t_ms = sum(prof[f]["ms"] for f in fams if f in prof)
+        fl = sum(prof[f]["flops"] for f in fams if f in prof)
+        rate = fl / max(t_ms * 1e-3, 1e-12)
+        return {"kernel": kernel, "achieved": round(rate / 1e12, 3), "peak": round(PEAK_SPLIT_MFMA / 1e12, 1),
+                "unit": "TFLOP/s", "frac": round(rate / PEAK_SPLIT_MFMA, 4), "ms_per_step": round(t_ms / n, 3),
+                "flop_per_step": fl / n}
+
     conv_fams = {k: v for k, v in prof.items() if k in GEMM_FAMS}
     gemm_ms = sum(v["ms"] for v in conv_fams.values())
     gemm_flops = sum(v["flops"] for v in conv_fams.values())
@@ -527,16 +544,16 @@ def main(argv=None):
     tpath = os.path.join(ROOT, "profiles", "hbm_traffic.json")
     if os.path.exists(tpath):  # measured HBM bytes per launch (rocprofv3 FETCH_SIZE / WRITE_SIZE passes)
         with open(tpath) as f:
-            traffic = json.load(f).get("conv_gemm", {}).get("bytes_per_launch")
-    wg = prof.get("conv_wgrad", {"ms": 0, "flops": 0, "launches": 0})
-    wgt = prof.get("convt_wgrad", {"ms": 0, "flops": 0, "launches": 0})
+            traffic = json.load(f).get("conv_fwd", {}).get("bytes_per_launch")
+    grads = {k: grad_roofline(prof, k, a.steps) for k in GRAD_FAMS}
+    grad_flops = sum(v["flop_per_step"] for v in grads.values()) * a.steps
     achieved = gemm_flops / (gemm_ms * 1e-3) if gemm_ms else 0.0
-    total_conv_flops = gemm_flops + wg["flops"] + wgt["flops"]
-    # step roofline: every conv FLOP at the FP32-MFMA peak plus the compulsory
-    # elementwise bytes (8 B/elem forward, 12 B/elem backward over the AdaIN
+    total_conv_flops = gemm_flops + grad_flops
+    # step roofline: every conv FLOP at its unit's peak (forwards FP32, grads
+    # split bf16) plus the compulsory elementwise bytes (8 B/elem forward, 12 B/elem backward over the AdaIN
     # units' elements) at the HBM peak
     elems = adain_elements(cfg, T) * B
-    ideal_s = (total_conv_flops / a.steps) / PEAK_FP32_MFMA + 20.0 * elems / PEAK_HBM
+    ideal_s = (gemm_flops / PEAK_FP32_MFMA + grad_flops / PEAK_SPLIT_MFMA) / a.steps + 20.0 * elems / PEAK_HBM
     out = {
         "metric": "Kokoro decoder fwd+bwd audio-sec/s (T=512,B=8); % of FP32-MFMA/HBM roofline",
         "value": round(value, 3),
@@ -554,7 +571,7 @@ def main(argv=None):
                                "iSTFT backward, with conv/convT/pool/fc weight grads, Snake alpha grads, d(style)",
                    "batch": B, "T": T, "audio_s_per_utterance": lens["audio_seconds"],
                    "audio_s_per_step": audio_per_step, "params": int(sum(np.prod(s) for s in shapes.values()))},
-        "roofline": {"bound": "mfma", "kernel": "conv_gemm (conv1d fwd / dgrad, convT fwd / dgrad)",
+        "roofline": {"bound": "mfma", "kernel": "conv_gemm_q, conv_gemm, corr_gemm (conv1d and convT forwards)",
                      "achieved": round(achieved / 1e12, 3), "peak": PEAK_FP32_MFMA / 1e12, "unit": "TFLOP/s",
                      "frac": round(achieved / PEAK_FP32_MFMA, 4), "traffic": traffic,
                      "region": "profiled pass of the same K steps (events around every family launch)",
@@ -562,9 +579,7 @@ def main(argv=None):
                      "launches_per_step": gemm_launches // a.steps,
                      "ms_per_step": round(gemm_ms / a.steps, 3),
                      "flop_per_step": gemm_flops / a.steps},
-        "wgrad_roofline": {"kernel": "wgrad_gemm", "achieved": round(
-            (wg["flops"] + wgt["flops"]) / max((wg["ms"] + wgt["ms"]) * 1e-3, 1e-12) / 1e12, 3),
-            "unit": "TFLOP/s", "ms_per_step": round((wg["ms"] + wgt["ms"]) / a.steps, 3)},
+        **grads,
         "step_roofline": {"ideal_ms": round(ideal_s * 1e3, 3), "frac": round(ideal_s * 1e3 / ms, 4),
                           "conv_tflop_per_step": round(total_conv_flops / a.steps / 1e12, 4),
                           "elementwise_gb_per_step": round(20.0 * elems / 1e9, 3)},
@@ -577,22 +592,16 @@ def main(argv=None):
         sp, n = serial.pop("prof"), serial["steps"]
         s_ms = sum(v["ms"] for k, v in sp.items() if k in GEMM_FAMS)
         s_fl = sum(v["flops"] for k, v in sp.items() if k in GEMM_FAMS)
-        swg = [sp.get(k, {"ms": 0, "flops": 0}) for k in ("conv_wgrad", "convt_wgrad")]
-        w_ms, w_fl = sum(v["ms"] for v in swg), sum(v["flops"] for v in swg)
         serial["roofline"] = {"kernel": out["roofline"]["kernel"], "achieved": round(s_fl / (s_ms * 1e-3) / 1e12, 3)
                               if s_ms else 0.0, "frac": round(s_fl / (s_ms * 1e-3) / PEAK_FP32_MFMA, 4) if s_ms else 0.0,
                               "ms_per_step": round(s_ms / n, 3)}
-        serial["wgrad_roofline"] = {"achieved": round(w_fl / max(w_ms * 1e-3, 1e-12) / 1e12, 3),
-                                    "frac": round(w_fl / max(w_ms * 1e-3, 1e-12) / PEAK_FP32_MFMA, 4),
-                                    "ms_per_step": round(w_ms / n, 3)}
+        serial.update({k: grad_roofline(sp, k, n) for k in GRAD_FAMS})
         serial["families_ms_per_step"] = {k: round(v["ms"] / n, 3) for k, v in sorted(sp.items())}
         out["serial"] = serial
         # The roofline figure is the one-stream pass's: there each conv GEMM
-        # launch has the GPU to itself, so the family's launch time per step
-        # stays within the step. On the default schedule up to three conv
-        # GEMMs and the weight-grad GEMMs share the CUs, each launch's
-        # duration also holds the others' work, and the family's summed
-        # launch time exceeds the step; that figure is kept, labelled.
+        # launch has the GPU to itself. On the default schedule up to three
+        # conv GEMMs share the CUs and each launch's duration also holds the
+        # others' work; that figure is kept, labelled.
         rf = out["roofline"]
         rf["frac_overlapped"], rf["achieved_overlapped"] = rf["frac"], rf["achieved"]
         rf["ms_per_step_overlapped"] = rf["ms_per_step"]
