@@ -8,20 +8,22 @@
 // rounds otherwise moves the gradients by up to 1e-3 (a few of 10^7 signs),
 // however small its own error.
 //
-// Forward family (one kernel, `conv_gemm`):
+// Forwards and input grads are one correlation,
 //   Y[n, m, q] = sum_{c, t} A[(c, t), m] * X[n, c, q*s + t*d - p]
-// with A the weights packed K-major ([C_in_pad * k][M_pad], zero padded so
-// tiles never test bounds on the A side). It serves
-//   - conv1d forward (A = W^T),
-//   - conv1d input-grad at stride 1 (A = the flipped transpose of W,
-//     p' = d(k-1) - p: the adjoint of a correlation is a correlation),
-//   - conv-transpose input-grad (a strided correlation of dY with W viewed as
-//     (C_in, C_out*k)),
+// with A the weights packed for the kernel that reads them, zero padded so
+// that tiles never test bounds on the A side:
+//   - conv1d forward (A = W^T): conv_gemm_q at stride 1 and k = 3, 7, 11,
+//     corr_gemm at stride 1 on grids of less than a round, conv_gemm else;
 //   - conv-transpose forward, polyphase: output phase r = (j + p) mod s sees
 //     only taps t = r + m*s, so each phase is a stride-1 correlation with
-//     ceil(k/s) taps whose outputs land at j = Q*s + r - p.
-// A 256-thread block owns a 128 (m) x 128 (q) output tile as 2x2 waves of
-// 64x64 (2x2 MFMA tiles each). Per K chunk the block stages CK input rows of
+//     ceil(k/s) taps whose outputs land at j = Q*s + r - p: corr_gemm on grids
+//     of less than a round, conv_gemm else;
+//   - conv1d input-grad at stride 1 (A = the flipped transpose of W,
+//     p' = d(k-1) - p: the adjoint of a correlation is a correlation) and
+//     conv-transpose input-grad (a strided correlation of dY with W viewed as
+//     (C_in, C_out*k)): split_gemm.
+// In conv_gemm a 256-thread block owns a 128 (m) x 128 (q) output tile as 2x2 waves
+// of 64x64 (2x2 MFMA tiles each). Per K chunk the block stages CK input rows of
 // the haloed window [q0*s - p, (q0+127)*s + (k-1)d - p] and the matching
 // CK*k weight rows in LDS; every tap then reads a shifted window of the same
 // staged rows, so X is fetched once per chunk instead of k times. Staging is
@@ -741,7 +743,8 @@ void conv_gemm(GemmArgs g) {
     constexpr int HS = CK / 2;
 
     // Two stages: chunk ch + 1 lands while ch is multiplied. One stage (where
-    // two would fit only two blocks per CU, the long strided windows): each
+    // two would fit only two blocks per CU, the windows of long strides and
+    // many taps: k = 20 at stride 10, not the decoder's k = 12 at 6): each
     // chunk is staged after every wave has read the previous one, and the
     // other resident blocks' MFMA work covers the wait.
     const bool single = g.single != 0;  // uniform
@@ -822,10 +825,10 @@ void conv_gemm(GemmArgs g) {
 #define CGQ_PF 2
 #endif
 // EPI picks the whole tiles' epilogue at compile time (split tiles always
-// store partials): QEPI_STORE the plain store, QEPI_ADAIN_BWD the AdaIN
-// backward row sums (store_tile_adain), QEPI_STATS the instance-norm moments
-// (store_tile_stats). One epilogue per instantiation keeps the live ranges of
-// the others out of the k-loop's register allocation.
+// store partials): QEPI_STORE the plain store, QEPI_STATS the instance-norm
+// moments (store_tile_stats; conv_gemm_q), QEPI_ADAIN_BWD the AdaIN backward
+// row sums (store_tile_adain; split_gemm). One epilogue per instantiation
+// keeps the live ranges of the others out of the k-loop's register allocation.
 enum { QEPI_STORE = 0, QEPI_ADAIN_BWD = 1, QEPI_STATS = 2 };
 
 // Where a conv_gemm_q tile stages its operands from (wave-uniform): the
@@ -1879,8 +1882,8 @@ __device__ inline long panel_index(int c, int t, int CK, int kk) {
 }
 
 // A[panel_index(c, t)][m] = W[m][c*k + t] (0 unless m < Mv and c < Cv): the
-// conv1d forward panel (m = co, c = ci) and the conv-transpose input-grad
-// panel (m = ci, c = co). A 32 (m) x 32 (j = c*k + t) tile passes through LDS:
+// conv1d forward panel of conv_gemm (m = co, c = ci). A 32 (m) x 32 (j = c*k +
+// t) tile passes through LDS:
 // W is read along its rows (j), A written along its rows (m). 32-square tiles
 // rather than 64: a single round of larger blocks spends most of its time
 // waiting on one load and one store round trip, and four times as many
@@ -3391,7 +3394,8 @@ static int wgrad_common(kdec_ctx* ctx, const float* X, long x_bs, const float* G
         return fail(ctx, KDEC_EINVAL, "wgrad: rows too long");
     if (static_cast<long>(M) * L_g * 4 > 0x7fffffffL || static_cast<long>(C_x) * L_x * 4 > 0x7fffffffL)
         return fail(ctx, KDEC_EINVAL, "wgrad: operand too large for one buffer descriptor");
-    {  // the longest input window that is taken: the rows of 128 (256) columns, KC positions each, in half of LDS
+    {  // the entry point's limit on a window, kept from one kernel to the next (this one runs any): the rows
+       // of 128 (256) columns, KC positions each, at 8 bytes in LDS
         const long NN = static_cast<long>(C_x) * k;
         const long bn = cdiv(NN, 128) * 128 < cdiv(NN, 256) * 256 ? 128 : 256;
         const long span = (KC - 1L) * s + (k - 1L) * d + 1;
@@ -3590,7 +3594,8 @@ int kdec_convt1d_dgrad(kdec_ctx* ctx, const float* W, const float* dY,
                "kdec_convt1d_dgrad: bad arguments");
     const int L_out = (L - 1) * stride - 2 * pad + (k - 1) + op + 1;
     KDEC_CHECK(ctx, L > 0 && L_out > 0, "kdec_convt1d_dgrad: empty output");
-    // what the strided correlation kernel takes: the same windows as the forward's
+    // the entry point's limits on a window, kept from one kernel to the next (split_gemm runs any): those of a
+    // strided forward of this k and stride
     const int CK = pick_ck(k, stride, 1);
     KDEC_CHECK(ctx, CK * k <= 64, "conv: bad chunk geometry");
     KDEC_CHECK(ctx, conv_lds_bytes(CK, k, stride, 1) <= 160 * 1024, "conv: tile does not fit LDS");

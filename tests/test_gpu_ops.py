@@ -139,10 +139,11 @@ def test_conv1d_wgrad_split_plans(K, C_out, L):
 
 @pytest.mark.parametrize("k,d", [(7, 3), (3, 1)])
 def test_conv1d_grid_beyond_one_round(K, k, d):
-    # 1301 output tiles: more than one round of resident blocks, so the last
-    # tiles run as channel-chunk parts reduced by tile_reduce while the others
-    # run whole. Reference: torch's float64 conv1d on the CPU (the C oracle
-    # covers the same kernel at the small sizes above).
+    # 1301 output tiles: more than one round of resident blocks, so the
+    # forward's last tiles run as channel-chunk parts reduced by tile_reduce
+    # while the others run whole (the input grad's all run whole: its parts are
+    # test_gpu_split.py's test_dgrad_parts). Reference: torch's float64 conv1d
+    # on the CPU (the C oracle covers the same kernel at the small sizes above).
     N, C_in, C_out, L = 1, 32, 128, 128 * 1300 + 1
     p = d * (k - 1) // 2
     x, W, b = rnd(N, C_in, L), rnd(C_out, C_in * k, scale=0.2), rnd(C_out)
@@ -227,11 +228,12 @@ def test_conv1d_fwd_stats(K, case):
 def test_conv1d_dgrad_adain_bwd_fused(K, case):
     # kdec_conv1d_dgrad_adain_bwd against the two calls it replaces
     # (kdec_conv1d_dgrad, then kdec_adain_act_bwd, each checked against the
-    # oracle elsewhere): the quad-packed GEMM with the AdaIN epilogue on whole
-    # tiles (C = 128, 1400 tiles, Snake, residual grad R), with split tail
-    # tiles reduced by tile_reduce_adain (C = 256: two output-channel tiles,
-    # leaky), and the unfused fallback on a small grid. dX, dgamma, dbeta and
-    # dalpha (accumulated onto a nonzero start) agree to summation order.
+    # oracle elsewhere): the GEMM with the AdaIN epilogue on whole tiles (C =
+    # 128, 1400 tiles, Snake, residual grad R; C = 256, 1320 tiles in two
+    # output-channel tiles, leaky), and the two calls on a small grid (tiles in
+    # parts are test_gpu_split.py's test_dgrad_adain_bwd_parts). dX, dgamma,
+    # dbeta and dalpha (accumulated onto a nonzero start) agree to summation
+    # order.
     N, C, Co, L, k, d, act, with_r = {
         "quad_snake_residual": (2, 128, 128, 128 * 700, 11, 5, "snake", True),
         "split_tiles_leaky": (2, 256, 256, 128 * 330 - 9, 7, 3, "leaky", False),
@@ -274,8 +276,10 @@ def test_conv1d_dgrad_adain_bwd_fused(K, case):
 @pytest.mark.parametrize("k,d", [(3, 5), (11, 1)])
 def test_conv1d_small_grid_split_parts(K, k, d):
     # 200 (forward) and 400 (input-grad) output tiles: fewer than one round of
-    # resident blocks, so every tile runs as channel-chunk parts (octet chunks
-    # of up to four taps) summed by tile_reduce. Reference: torch float64.
+    # resident blocks. The forward's tiles run their channel-chunk parts one
+    # after the other in a block, the input grad's run whole (parts in blocks of
+    # their own: test_gpu_small_grids.py's test_conv_fwd_parts, test_dgrad_parts).
+    # Reference: torch float64.
     N, C_in, C_out, L = 2, 256, 128, 128 * 100 - 7
     p = d * (k - 1) // 2
     x, W, b = rnd(N, C_in, L), rnd(C_out, C_in * k, scale=0.1), rnd(C_out)

@@ -71,6 +71,18 @@ def test_conv_fwd_parts(K):
     assert rel(y, 0.5 * (ref + r.double()) + 2.0 * y0.double()) <= TOL
 
 
+@pytest.mark.parametrize("N,ci,co,L,k,s", [(2, 33, 130, 2600, 20, 10), (1, 5, 7, 5200, 32, 16)])
+def test_conv_fwd_long_strides(K, N, ci, co, L, k, s):
+    # strided windows of which two stages leave two blocks per CU: staged once
+    g = torch.Generator().manual_seed(k)
+    p = (k - s) // 2
+    Lo = (L + 2 * p - k) // s + 1
+    x, w, b = torch.randn(N, ci, L, generator=g), torch.randn(co, ci * k, generator=g), torch.randn(co, generator=g)
+    xg, wg, bg, y = x.cuda(), w.cuda(), b.cuda(), torch.full((N, co, Lo), 7.0, device="cuda")
+    K.call("kdec_conv1d_fwd", P(xg), ci * L, P(wg), P(bg), P(y), co * Lo, N, ci, L, co, k, s, p, 1, None, 0, 1.0, 0.0)
+    assert rel(y, F.conv1d(x.double(), w.double().reshape(co, ci, k), b.double(), stride=s, padding=p)) <= TOL
+
+
 @pytest.mark.parametrize("k,s,L", [(20, 10, 42), (20, 10, 400), (12, 6, 4000), (3, 4, 9), (5, 1, 140)])
 def test_convt_fwd_edges(K, k, s, L):
     N, ci, co, p = 1, 72, 136, max(0, (k - s) // 2)
